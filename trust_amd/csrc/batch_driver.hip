@@ -159,6 +159,7 @@ int enqueue_segments(Ctx *ctx, const trust_params &p, int mode, const ResidentRu
             const int32_t *loc = sb + q.beg_off;
             const int32_t *glo = sb + (q.beg_off - q.v0);
             CsrViews v{loc, adj + q.e0, loc, adj + q.e0, glo, adj + q.e0};
+            v.ids = g.V;
             SegView sv;
             sv.list = (const int32_t *)ctx->list.p + q.v0;
             sv.graph_vbase = (const long long *)ctx->seg_vbase.p + q.vbase_off;
@@ -189,6 +190,8 @@ int read_ctl(Ctx *ctx, const ResidentRun &R, TcCtl &h)
     HIPCHK(hipMemcpyAsync(hs.data(), ctx->ctl.p, sizeof(TcCtl) * n, hipMemcpyDeviceToHost,
                           ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    for (TcCtl &x : hs)
+        fold_ctl(x);
     h = hs[0];
     for (size_t k = 1; k < n; k++) {  // list_begin is summed too: tier sizes are its differences
         h.count += hs[k].count;

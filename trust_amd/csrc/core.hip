@@ -500,7 +500,7 @@ core_dense_kernel(const DenseRec<OffT> *__restrict__ recs, long long cap,
     }
     acc = wave_sum(acc);
     if (lane == 0 && acc)
-        atomicAdd(&ctl->count, acc);
+        atomicAdd(&ctl->sums[blockIdx.x % kSumLines].count, acc);
 }
 
 // ------------------------------------------------------------------ host

@@ -51,6 +51,8 @@ struct CsrViews {
     // walk entries as WalkEntry<OffT> (list start and length; null: adjW
     // holds ids)
     const void *entW = nullptr;
+    // ids of the hash and probe rows are below this
+    int64_t ids = int64_t(1) << 31;
 };
 
 // Shape of one counting launch.
@@ -107,7 +109,6 @@ struct WiSlice {
 
 // C2's work queue of the binned walk-index build (walk_index.hip): chunks
 // of a slice's records, in one list per XCD.
-constexpr int kXcds = 8;
 struct WiChunk {
     int slice;
     int pad;

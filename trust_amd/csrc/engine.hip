@@ -165,14 +165,13 @@ int resolve_launch(Ctx *ctx, const trust_params &p, int64_t max_deg_hash, int64_
     int rc = shape_occupancy(ctx, m, off64, p.blocks, mode, false);
     if (rc)
         return rc;
+    if (p.blocks <= 0)  // no workgroup without a vertex
+        m.blocks = (int)std::min<int64_t>(m.blocks, std::max<int64_t>(V, 1));
     if (p.chunk > 0) {
         L.chunk_group = L.chunk_wave = p.chunk;
     } else {
-        // about 16 grabs per wave, at most 32 vertices each (large chunks of
-        // a skewed list leave long chunks for the end)
         L.chunk_group = 1;
-        const long long waves = (long long)m.blocks * nwaves;
-        L.chunk_wave = (int)std::max<long long>(1, std::min<long long>(32, V / (waves * 16 + 1)));
+        L.chunk_wave = 0;  // by the kernel, from the tier's vertices
     }
     // large-LDS launch for tables the main launch cannot hold, plus the
     // HBM-table tier for tables no LDS can hold
@@ -240,6 +239,8 @@ static void fill_args(TcArgs<OffT> &a, Ctx *ctx, const CsrViews &views, const tr
     a.nranks = p.total_process;
     a.force_linear = (p.flags & TRUST_FLAG_LINEAR_PROBING) ? 1
                      : (p.flags & TRUST_FLAG_REBUILD_LINEAR) ? 2 : 0;
+    if (!a.force_linear)  // a pack has no linear-probing form
+        pack_limits(views.ids, s.wave_lg, &a.pack_rows, &a.tag_shift);
     a.ctl = ctl_dev;
     a.instr_cycles = instr_cycles;
     a.instr_probes = instr_probes;
@@ -753,6 +754,7 @@ int enqueue_resident(Ctx *ctx, const trust_params &p, int mode, const ResidentRu
         return enqueue_segments(ctx, p, mode, R, timed);
     CsrViews v{g.beg.p, (const int32_t *)g.adj.p, g.beg.p, (const int32_t *)g.adj.p, g.beg.p,
                (const int32_t *)g.adj.p};
+    v.ids = g.V;
     if (timed)
         HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
     int rc;

@@ -26,8 +26,8 @@ namespace trust {
 
 constexpr int64_t kNoAllocMaxV = int64_t(1) << 22;
 constexpr size_t kScrCtl = 0;                      // TcCtl
-constexpr size_t kScrMisc = 4096;                  // NoAllocMisc
-constexpr size_t kScrBlocks = 8192;                // kNumTiers x planner blocks (long long)
+constexpr size_t kScrMisc = 16384;                 // NoAllocMisc
+constexpr size_t kScrBlocks = 20480;               // kNumTiers x planner blocks (long long)
 constexpr size_t kScrBlocksBytes = sizeof(long long) * kNumTiers *
                                    ((kNoAllocMaxV + kPlanPerBlock - 1) / kPlanPerBlock);
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -222,6 +222,8 @@ extern "C" int trust_count_csr_noalloc(const int64_t *beg_dev, const int32_t *ad
     a.nranks = p->total_process;
     a.force_linear = (p->flags & TRUST_FLAG_LINEAR_PROBING) ? 1
                      : (p->flags & TRUST_FLAG_REBUILD_LINEAR) ? 2 : 0;
+    if (!a.force_linear)
+        pack_limits(V, L.main.wave_lg, &a.pack_rows, &a.tag_shift);
     a.ctl = ctl;
     if (L.has_big) {  // tables beyond the main launch's LDS share
         a.table_words = L.big.table_words;
@@ -244,9 +246,10 @@ extern "C" int trust_count_csr_noalloc(const int64_t *beg_dev, const int32_t *ad
     hipLaunchKernelGGL(na_stamp_kernel, dim3(1), dim3(1), 0, s, &misc->t1);
     HIPCHK(hipGetLastError());
     TcCtl h;
-    HIPCHK(hipMemcpyAsync(&h, ctl, sizeof(h), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(&h, ctl, kCtlHead, hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(&hm, misc, sizeof(hm), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
+    fold_ctl(h);
     if (h.list_begin[kTierSpill + 1] != h.list_begin[kTierSpill])
         return fail(TRUST_ERR_OVERFLOW, "a table needs HBM, which the allocation-free path lacks");
     if (r) {

@@ -398,6 +398,7 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
                 return hip_fail(e, "journal event");
             unsigned long long c = 0, w = 0;
             for (int q = 0; q < per_job; q++) {
+                fold_ctl(hctl[(size_t)(per_job * job + q)]);
                 c += hctl[(size_t)(per_job * job + q)].count;
                 w += hctl[(size_t)(per_job * job + q)].probes;
             }
@@ -585,6 +586,9 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
     std::vector<TcCtl> h((size_t)nctl);
     HIPCHK(hipMemcpyAsync(h.data(), ctls.p, sizeof(TcCtl) * (size_t)nctl, hipMemcpyDeviceToHost,
                           ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    for (TcCtl &x : h)
+        fold_ctl(x);
     if (short_walk)  // fold each job's in-walk count into its out-walk count
         for (long long j : todo) {
             TcCtl &a = h[(size_t)(2 * j)];
@@ -593,7 +597,6 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
             a.probes += b.probes;
             a.rebuilds += b.rebuilds;
         }
-    HIPCHK(hipStreamSynchronize(ctx->stream));
     if (journal && (rc = journal_ready(true)))
         return rc;
     float ms = 0;
@@ -786,6 +789,7 @@ extern "C" int trust_triangle_count_partition(int rank, const char *folder, int 
     TcCtl h;
     HIPCHK(hipMemcpyAsync(&h, ctx.ctl.p, sizeof(TcCtl), hipMemcpyDeviceToHost, ctx.stream));
     HIPCHK(hipStreamSynchronize(ctx.stream));
+    fold_ctl(h);
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, ctx.ev[0], ctx.ev[2]));
     for (int q = 0; q < 3; q++) {

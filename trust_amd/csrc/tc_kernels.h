@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace trust {
@@ -40,20 +41,44 @@ constexpr int kProbeDeep = 16;
 
 // Device control block: queue cursors, list bounds and results.  Cleared
 // by a fill kernel before a run.
-// The wave queue is split over kQueueShards counters, each on its own
-// 128-byte line: one address sustains only about 1e8 atomics/s, which
-// bounds graphs of many small vertices.
-constexpr int kQueueShards = 8;
+//
+// Each work queue is split over several counters, each on its own 128-byte
+// line: one address sustains only about 87 M atomics/s (11.5 ns each), and a
+// line that many waves wait for also holds up the other accesses of its
+// memory channel (in a count of R-MAT 16, whose 38k vertices take an atomic
+// each, vertices of two neighbours took 13 us at the end of a launch).  The
+// workgroup tiers hand out 8, the wave tier 32 shards.
+constexpr int kXcds = 8;  // each with its own L2
+constexpr int kWaveShards = 32;
+constexpr int kGroupShards = 8;
 constexpr int kShardStride = 32;  // unsigned ints per counter line
-struct TcCtl {
-    unsigned long long count;       // triangles
-    unsigned long long probes;      // hash lookups (W)
-    unsigned int next[8];           // queue cursors, one per tier
+// The results are summed per workgroup and added to one of kSumLines lines,
+// for the same reason: 8192 waves adding to one count and one probe total
+// took 190 us at the end of a launch in which every wave had work.
+constexpr int kSumLines = 16;
+struct alignas(128) TcSum {
+    unsigned long long count, probes;
+};
+struct alignas(128) TcCtl {
+    unsigned long long count;       // triangles       (totals: host side,
+    unsigned long long probes;      // hash lookups (W) fold_ctl)
     long long list_begin[8];        // tier t occupies list[list_begin[t], list_begin[t+1])
     unsigned long long rebuilds;    // tables rebuilt with linear probing after a cuckoo attempt
-    unsigned long long pad[3];
-    unsigned int shard[kQueueShards * kShardStride];  // wave-queue cursors
+    TcSum sums[kSumLines];          // triangles and hash lookups, by workgroup
+    // queue cursors (a copy to the host needs none of what follows: kCtlHead)
+    alignas(128) unsigned int wave_next[kWaveShards * kShardStride];
+    unsigned int group_next[kTierWave][kGroupShards * kShardStride];  // by tier
 };
+// Bytes of a control block that hold results (list bounds, sums).
+constexpr size_t kCtlHead = offsetof(TcCtl, wave_next);
+// Totals of a control block copied back to the host.
+inline void fold_ctl(TcCtl &h)
+{
+    for (const TcSum &x : h.sums) {
+        h.count += x.count;
+        h.probes += x.probes;
+    }
+}
 
 // Three CSR views: the hash source (N+(u) that is tabled), the walk (the v
 // in N+(u) whose lists are probed) and the probe rows (N+(v)).  For an
@@ -88,7 +113,9 @@ struct TcArgs {
     int wave_slots;          // LDS ints per wave table
     int wave_lg;
     int chunk_group;         // vertices per grab, spill/group tiers
-    int chunk_wave;          // vertices per grab, wave tier
+    int chunk_wave;          // vertices per grab, wave tier (0: chosen by the kernel)
+    int pack_rows;           // rows a pack of the wave tier may hold (0, 1: no packs)
+    int tag_shift;           // bits of an id (a pack's keys are id | row << tag_shift)
     int rank;
     int nranks;
     int force_linear;        // 1: linear-probing tables only (no cuckoo); 2: every cuckoo
@@ -186,9 +213,23 @@ hipError_t launch_side_stats(const OffT *beg, const int32_t *adj, long long V,
 // more; measured break-even near 0.45-0.5 on R-MAT).
 constexpr double kShortWalkShare = 0.45;
 
+// Packs of the wave tier (tc_kernels.hip): ids below `ids` leave the upper
+// bits of a 32-bit key for the row's number; the largest number is left out,
+// since with all ids' bits set it would be the empty slot's mark.
+inline void pack_limits(long long ids, int wave_lg, int *rows, int *shift)
+{
+    int bits = 1;
+    while (bits < 31 && (1ll << bits) < ids)
+        bits++;
+    *shift = bits;
+    const long long most = (1ll << (32 - bits)) - 1;
+    // a pack holds up to 64 keys: its table needs 128 slots
+    *rows = wave_lg < 7 || most < 2 ? 0 : most < kWave ? (int)most : kWave;
+}
+
 // Per-wave LDS ints after the tables: a 64-int mark array, then the wave's
 // graph state of the batch mode.
-constexpr int kMarkStride = kWave + 4;
+constexpr int kMarkStride = kWave + 8;
 // LDS ints besides the tables: per-wave marks, misc words, chunk totals.
 inline int lds_extra_words(int threads)
 {

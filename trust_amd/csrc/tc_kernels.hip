@@ -44,15 +44,24 @@ namespace trust {
 constexpr int kEmpty = -1;
 constexpr int kNoProbe = -2;  // a window position past the end: matches no slot
 
-// Per-wave attribution of triangles to the graphs of a batch.  The state
-// sits in LDS, in the kMarkStride - kWave words after the wave's mark array
-// (gs[0], gs[1]) = the vertex range of the graph being counted, gs[2] = that
-// graph (-1: none), not in scalar registers, where it would stay live across
-// the whole probe walk and push other values out.  The wave's running count
-// acc holds the current graph's triangles only: entering a vertex of another
-// graph adds acc to the previous graph, with a completion time stamp, and
-// clears it.  Called with the whole wave active, u wave-uniform, before the
-// vertex's hits are added to acc.
+// The kernel's arguments, read through the kernel argument segment.  The
+// fields are wave-uniform and loaded with scalar loads; held by value they
+// stay in scalar registers across the whole probe walk, and the count kernel
+// spilled 80-124 of them (into vector registers, which then spilled too).
+// A pointer from args_again() hides that it is the same one, so a workgroup
+// vertex loads the fields it needs afresh (from the scalar cache).  The wave
+// tier's vertices are too short for that: their loads would wait for these.
+template <typename OffT>
+using ArgP = const __attribute__((address_space(4))) TcArgs<OffT> *;
+
+template <typename OffT>
+__device__ __forceinline__ ArgP<OffT> args_again()
+{
+    auto p = (ArgP<OffT>)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 __device__ __forceinline__ unsigned long long uniform(unsigned long long x)
 {
     const int lo = __builtin_amdgcn_readfirstlane((int)(x & 0xffffffffu));
@@ -60,48 +69,76 @@ __device__ __forceinline__ unsigned long long uniform(unsigned long long x)
     return ((unsigned long long)(unsigned int)hi << 32) | (unsigned int)lo;
 }
 
+// Per-wave attribution of triangles to the graphs of a batch.  The state
+// sits in LDS, in the kMarkStride - kWave words after the wave's mark array,
+// not in registers, where it would stay live across the whole probe walk and
+// push other values out: (gs[0], gs[1]) = the vertex range of the graph being
+// counted, gs[2] = that graph (-1: none), gs[4..5] = its triangles so far.
+// Entering a vertex of another graph adds those to the previous graph, with
+// a completion time stamp, and clears them.  Called with the whole wave
+// active, u wave-uniform, before the vertex's hits are added.
 __device__ __forceinline__ void graph_init(int *gs)
 {
-    gs[0] = 0;
-    gs[1] = 0;  // an empty range: the first vertex enters its graph
-    gs[2] = -1;
+    if (lane_id() < kMarkStride - kWave)
+        gs[lane_id()] = lane_id() == 2 ? -1 : 0;  // an empty range: the first vertex enters its graph
+    wave_sync();
 }
 
 template <typename Args>
-__device__ __forceinline__ void graph_flush(const Args &a, int *gs, unsigned long long &acc)
+__device__ __forceinline__ void graph_flush(Args a, int *gs)
 {
-    const unsigned long long total = uniform(wave_sum(acc));
     const int g = __builtin_amdgcn_readfirstlane(gs[2]);
-    if (g >= 0 && __lane_id() == 0) {
-        if (total)
-            atomicAdd(a.graph_counts + g, total);
-        atomicMax(a.graph_done + g, (unsigned long long)wall_clock64());
+    if (g >= 0 && lane_id() == 0) {
+        unsigned long long *total = (unsigned long long *)(gs + 4);
+        if (*total)
+            atomicAdd(a->graph_counts + g, *total);
+        atomicMax(a->graph_done + g, (unsigned long long)wall_clock64());
+        *total = 0;
     }
-    acc = 0;
+    wave_sync();
 }
 
 template <typename Args>
-__device__ __forceinline__ void graph_enter(const Args &a, int *gs, int u,
-                                            unsigned long long &acc)
+__device__ __forceinline__ void graph_enter(Args a, int *gs, int u)
 {
     const int2 range = *(const int2 *)gs;
     if (u >= __builtin_amdgcn_readfirstlane(range.x) && u < __builtin_amdgcn_readfirstlane(range.y))
         return;
-    graph_flush(a, gs, acc);
+    graph_flush(a, gs);
     // the page of u bounds the search: vbase[lo] <= u < vbase[hi]
-    const int pg = u >> a.graph_page_shift;
-    int lo = a.graph_page[pg], hi = a.graph_page[pg + 1] + 1;
+    const int pg = u >> a->graph_page_shift;
+    int lo = a->graph_page[pg], hi = a->graph_page[pg + 1] + 1;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
-        if (a.graph_vbase[mid] <= u)
+        if (a->graph_vbase[mid] <= u)
             lo = mid;
         else
             hi = mid;
     }
     const int g = __builtin_amdgcn_readfirstlane(lo);
-    gs[0] = (int)a.graph_vbase[g];  // every lane stores the same values
-    gs[1] = (int)a.graph_vbase[g + 1];
+    gs[0] = (int)a->graph_vbase[g];  // every lane stores the same values
+    gs[1] = (int)a->graph_vbase[g + 1];
     gs[2] = g;
+    wave_sync();
+}
+
+// Adds a wave's hits and probes of one vertex (wave-uniform) to the sums in
+// LDS: the workgroup's {triangles, probes}, in batch mode the triangles to
+// the wave's current graph.
+template <int kMode>
+__device__ __forceinline__ void add_result(unsigned long long *sum, int *mark,
+                                           unsigned long long hits, unsigned long long probes)
+{
+    const int lane = lane_id();
+    if constexpr (kMode == kModeBatch) {
+        if (lane == 0)
+            *(unsigned long long *)(mark + kWave + 4) += hits;
+        if (lane == 1)
+            atomicAdd(sum + 1, probes);
+    } else {
+        if (lane < 2)
+            atomicAdd(sum + lane, lane == 0 ? hits : probes);
+    }
 }
 
 // ---------------------------------------------------------- hash tables
@@ -320,19 +357,19 @@ __device__ __forceinline__ Group<OffT> load_group(int v, bool valid, const OffT 
 // place, coalesced, one load per entry; otherwise the entry is a vertex id whose offsets
 // are looked up.
 template <typename OffT>
-__device__ __forceinline__ Group<OffT> walk_group(const TcArgs<OffT> &a, OffT at, bool valid)
+__device__ __forceinline__ Group<OffT> walk_group(ArgP<OffT> a, OffT at, bool valid)
 {
-    if (a.entW) {
+    if (a->entW) {
         OffT s = 0;
         int deg = 0;
         if (valid) {
-            const WalkEntry<OffT> x = a.entW[at];
+            const WalkEntry<OffT> x = a->entW[at];
             s = x.start;
             deg = x.deg;
         }
         return make_group(s, deg);
     }
-    return load_group(valid ? a.adjW[at] : 0, valid, a.begP);
+    return load_group(valid ? a->adjW[at] : 0, valid, a->begP);
 }
 
 // Probes windows [wbeg, wend) (64 positions each) of a group's
@@ -483,42 +520,43 @@ __device__ __forceinline__ unsigned long long probe_windows(const Group<OffT> &g
 // capacity 2^cap_lg.  misc[0]: unit cursor, misc[2]: window total;
 // ctot: kMaxChunks+1 ints of LDS.
 template <typename OffT, bool kGlobal, int kMode, int kU>
-__device__ __forceinline__ void group_vertex(const TcArgs<OffT> &a, int u, int *tab, int cap_lg,
-                                             int *mark, int *misc, int *ctot,
-                                             unsigned long long &acc, unsigned long long &probes)
+__device__ __forceinline__ void group_vertex(int u, int *tab, int cap_lg,
+                                             int *mark, int *misc, int *ctot)
 {
     constexpr bool kInstr = kMode == kModeInstr;
     constexpr bool kTable = kMode != kModeGather;
+    ArgP<OffT> a = args_again<OffT>();
     if constexpr (kMode == kModeBatch)
-        graph_enter(a, mark + kWave, u, acc);
+        graph_enter(a, mark + kWave, u);
     unsigned long long t0 = 0;
     if (kInstr && threadIdx.x == 0)
         t0 = clock64();
     const int lane = lane_id();
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);  // uniform
+    const int tid = wave * kWave + lane;
     const int nwaves = blockDim.x / kWave;
-    const OffT sH = a.begH[u];
-    const int dH = (int)(a.begH[u + 1] - sH);
-    const OffT sW = a.begW[u];
-    const int dW = (int)(a.endW[u] - sW);
+    const OffT sH = a->begH[u];
+    const int dH = (int)(a->begH[u + 1] - sH);
+    const OffT sW = a->begW[u];
+    const int dW = (int)(a->endW[u] - sW);
     const int lg = table_lg(dH, cap_lg);
     const int size = 1 << lg;
     if constexpr (kTable)
-        for (int i = threadIdx.x; i < size; i += blockDim.x)
+        for (int i = tid; i < size; i += blockDim.x)
             slot_clear<kGlobal>(tab + i);
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         misc[0] = 0;                       // window-unit cursor
-        misc[3] = a.force_linear == 1;     // linear-probing table for this vertex
+        misc[3] = a->force_linear == 1;     // linear-probing table for this vertex
     }
     if constexpr (kGlobal)
         __threadfence();  // HBM slots: cleared values visible in L2 before any insert/lookup
     __syncthreads();
     bool linear = false;
     if constexpr (kTable) {
-        bool failed = a.force_linear == 2;  // forced: rebuild after the cuckoo attempt
-        if (a.force_linear != 1)
-            for (int i = threadIdx.x; i < dH; i += blockDim.x)
-                failed |= cuckoo_insert(tab, lg - 1, a.adjH[sH + (OffT)i]);
+        bool failed = a->force_linear == 2;  // forced: rebuild after the cuckoo attempt
+        if (a->force_linear != 1)
+            for (int i = tid; i < dH; i += blockDim.x)
+                failed |= cuckoo_insert(tab, lg - 1, a->adjH[sH + (OffT)i]);
         if (failed)
             misc[3] = 1;  // benign race: every writer stores 1
         if constexpr (kGlobal)
@@ -526,21 +564,22 @@ __device__ __forceinline__ void group_vertex(const TcArgs<OffT> &a, int u, int *
         __syncthreads();
         linear = misc[3] != 0;
         if (linear) {  // rebuild this vertex's table with linear probing
-            if (threadIdx.x == 0 && a.force_linear != 1)
-                atomicAdd(&a.ctl->rebuilds, 1ull);
+            if (tid == 0 && a->force_linear != 1)
+                atomicAdd(&a->ctl->rebuilds, 1ull);
             __syncthreads();
-            for (int i = threadIdx.x; i < size; i += blockDim.x)
+            for (int i = tid; i < size; i += blockDim.x)
                 slot_clear<kGlobal>(tab + i);
             if constexpr (kGlobal)
                 __threadfence();
             __syncthreads();
-            for (int i = threadIdx.x; i < dH; i += blockDim.x)
-                table_insert(tab, lg, a.adjH[sH + (OffT)i]);
+            for (int i = tid; i < dH; i += blockDim.x)
+                table_insert(tab, lg, a->adjH[sH + (OffT)i]);
         }
     }
     if constexpr (kGlobal)
         __threadfence();
     __syncthreads();
+    a = args_again<OffT>();
     const int nchunks = (dW + kWave - 1) / kWave;
     unsigned long long hits = 0;  // wave-uniform
     unsigned long long wave_probes = 0;
@@ -600,7 +639,7 @@ __device__ __forceinline__ void group_vertex(const TcArgs<OffT> &a, int u, int *
                     cur = lo;
                 }
                 const int cend = min(w1, ctot[lo + 1]);
-                hits += probe_windows<OffT, kGlobal, kMode, kU>(g, w0 - ctot[lo], cend - ctot[lo], a.adjP,
+                hits += probe_windows<OffT, kGlobal, kMode, kU>(g, w0 - ctot[lo], cend - ctot[lo], a->adjP,
                                                      tab, lg, linear, mark);
                 w0 = cend;
             }
@@ -617,70 +656,63 @@ __device__ __forceinline__ void group_vertex(const TcArgs<OffT> &a, int u, int *
             const int idx = c * kWave + lane;
             const Group<OffT> g = walk_group(a, sW + (OffT)idx, idx < dW);
             wave_probes += (unsigned long long)g.total;
-            hits += probe_windows<OffT, kGlobal, kMode, kU>(g, 0, (g.total + kWave - 1) / kWave, a.adjP, tab,
+            hits += probe_windows<OffT, kGlobal, kMode, kU>(g, 0, (g.total + kWave - 1) / kWave, a->adjP, tab,
                                                  lg, linear, mark);
         }
     }
-    acc += lane == 0 ? hits : 0ull;  // the wave's hits count once
-    probes += wave_probes;
+    add_result<kMode>((unsigned long long *)(misc + 4), mark, hits, wave_probes);
     __syncthreads();
     if constexpr (kInstr) {
         if (lane == 0 && wave_probes)
-            atomicAdd(a.instr_probes + u, wave_probes);
-        if (threadIdx.x == 0)
-            a.instr_cycles[u] = clock64() - t0;
+            atomicAdd(a->instr_probes + u, wave_probes);
+        if (tid == 0)
+            a->instr_cycles[u] = clock64() - t0;
     }
 }
 
 // One wavefront counts vertex u with its own LDS table slice.
 template <typename OffT, int kMode, int kU>
-__device__ __forceinline__ void wave_vertex(const TcArgs<OffT> &a, int u, int *tab, int *mark,
-                                            unsigned long long &acc, unsigned long long &probes)
+__device__ __forceinline__ void wave_vertex(ArgP<OffT> a, int u, OffT sH, int dH, OffT sW, int dW,
+                                            int *tab, int *mark, unsigned long long *sum)
 {
     constexpr bool kInstr = kMode == kModeInstr;
     constexpr bool kTable = kMode != kModeGather;
-    if constexpr (kMode == kModeBatch)
-        graph_enter(a, mark + kWave, u, acc);
     unsigned long long t0 = 0;
     if (kInstr)
         t0 = clock64();
     const int lane = lane_id();
-    const OffT sH = a.begH[u];
-    const int dH = (int)(a.begH[u + 1] - sH);
-    const OffT sW = a.begW[u];
-    const int dW = (int)(a.endW[u] - sW);
-    const int lg = table_lg(dH, a.wave_lg);
+    const int lg = table_lg(dH, a->wave_lg);
     const int size = 1 << lg;
     // On an unpartitioned graph the hashed row and the walked row are one
     // row: its first 64 ids, loaded for the table, also start the walk
     // (one dependent load less per vertex).
-    const bool same_row = kTable && a.adjH == a.adjW && sH == sW && dH == dW;
+    const bool same_row = kTable && a->adjH == a->adjW && sH == sW && dH == dW;
     int head = 0;
     if constexpr (kTable)
-        head = lane < dH ? a.adjH[sH + (OffT)lane] : 0;
+        head = lane < dH ? a->adjH[sH + (OffT)lane] : 0;
     bool linear = false;
     if constexpr (kTable) {
         for (int i = lane; i < size; i += kWave)
             tab[i] = kEmpty;
         wave_sync();
         // force_linear 1: linear probing only; 2: rebuild after the cuckoo attempt
-        bool failed = a.force_linear != 0;
-        if (a.force_linear != 1) {
+        bool failed = a->force_linear != 0;
+        if (a->force_linear != 1) {
             if (lane < dH)
                 failed |= cuckoo_insert(tab, lg - 1, head);
             for (int i = lane + kWave; i < dH; i += kWave)
-                failed |= cuckoo_insert(tab, lg - 1, a.adjH[sH + (OffT)i]);
+                failed |= cuckoo_insert(tab, lg - 1, a->adjH[sH + (OffT)i]);
         }
         wave_sync();
         linear = __ballot(failed) != 0;
         if (linear) {  // rebuild this vertex's table with linear probing
-            if (lane == 0 && a.force_linear != 1)
-                atomicAdd(&a.ctl->rebuilds, 1ull);
+            if (lane == 0 && a->force_linear != 1)
+                atomicAdd(&a->ctl->rebuilds, 1ull);
             for (int i = lane; i < size; i += kWave)
                 tab[i] = kEmpty;
             wave_sync();
             for (int i = lane; i < dH; i += kWave)
-                table_insert(tab, lg, a.adjH[sH + (OffT)i]);
+                table_insert(tab, lg, a->adjH[sH + (OffT)i]);
             wave_sync();
         }
     }
@@ -689,50 +721,336 @@ __device__ __forceinline__ void wave_vertex(const TcArgs<OffT> &a, int u, int *t
     for (int c = 0; c < dW; c += kWave) {
         const bool valid = c + lane < dW;
         Group<OffT> g;
-        if (a.entW) {
+        if (a->entW) {
             g = walk_group(a, sW + (OffT)(c + lane), valid);
         } else {
-            const int v = c == 0 && same_row ? head : (valid ? a.adjW[sW + (OffT)(c + lane)] : 0);
-            g = load_group(v, valid, a.begP);
+            const int v = c == 0 && same_row ? head : (valid ? a->adjW[sW + (OffT)(c + lane)] : 0);
+            g = load_group(v, valid, a->begP);
         }
         wave_probes += (unsigned long long)g.total;
-        hits += probe_windows<OffT, false, kMode, kU>(g, 0, (g.total + kWave - 1) / kWave, a.adjP, tab, lg,
+        hits += probe_windows<OffT, false, kMode, kU>(g, 0, (g.total + kWave - 1) / kWave, a->adjP, tab, lg,
                                            linear, mark);
     }
     wave_sync();
-    acc += lane == 0 ? hits : 0ull;  // the wave's hits count once
-    probes += wave_probes;
+    add_result<kMode>(sum, mark, hits, wave_probes);
     if constexpr (kInstr) {
         if (lane == 0) {
-            a.instr_probes[u] = wave_probes;
-            a.instr_cycles[u] = clock64() - t0;
+            a->instr_probes[u] = wave_probes;
+            a->instr_cycles[u] = clock64() - t0;
         }
     }
 }
 
-// ------------------------------------------------------------ the kernel
-template <typename OffT, int kMode, bool kGlobal, int kU>
-__device__ __forceinline__ void group_phase(const TcArgs<OffT> &a, int tier, int *tab, int cap_lg,
-                                            int *mark, int *misc, int *ctot,
-                                            unsigned long long &acc, unsigned long long &probes)
+// ------------------------------------------------------------------ packs
+// Vertices with short rows are counted several to a wave.  One at a time, a
+// vertex of five neighbours costs the wave its table, its scans, a partly
+// filled window or two and a chain of dependent loads, about 250
+// instructions: on Chung-Lu (4.4 neighbours, 37 probes per vertex) the count
+// was bound by issuing them.  Packs took it from 1.20 to 0.44 ms, and a batch
+// of 400 ER/BA graphs (18 neighbours, 306 probes) from 8.4 to 7.3 ms.  A pack is a run of list positions whose rows
+// hold at most 64 entries together: a lane per entry loads the ids, one
+// table holds the keys of every row, tagged with the row's number in the
+// pack, and the 64 probed lists are laid end to end as for one vertex, each
+// position looked up with the tag of its entry's row.
+//
+// Ids take tag_shift bits, so id | row << tag_shift is exact; rows stay
+// below pack_rows, which keeps every key off kEmpty and kNoProbe.  One id is
+// often in many rows of a pack (hubs are), so the buckets depend on the row
+// too.  A pack whose insertion fails is counted vertex by vertex.
+constexpr int kPackLg = 8;  // table of 2^kPackLg slots (>= 4 per key), at most the wave's slice
+
+__device__ __forceinline__ unsigned int pack_fold(unsigned int id, unsigned int row)
 {
-    const long long lb = a.ctl->list_begin[tier], le = a.ctl->list_begin[tier + 1];
-    if (le <= lb)
-        return;
-    for (;;) {
-        __syncthreads();
-        if (threadIdx.x == 0)
-            misc[1] = (int)atomicAdd(&a.ctl->next[tier], 1u);
-        __syncthreads();
-        const long long c = (long long)(unsigned int)misc[1] * a.nranks + a.rank;
-        const long long first = lb + c * a.chunk_group;
-        if (first >= le)
-            break;
-        const long long last = min(first + (long long)a.chunk_group, le);
-        for (long long i = first; i < last; i++)
-            group_vertex<OffT, kGlobal, kMode, kU>(a, a.list[i], tab, cap_lg, mark, misc, ctot, acc,
-                                                probes);
+    return id + __umul24(row, 0x9E5u);
+}
+
+// Inserts key = id | row << shift; true: not placed within kMaxKicks.
+__device__ __forceinline__ bool pack_insert(int *tab, int lgb, int key, int shift)
+{
+    for (int it = 0; it < kMaxKicks; it++) {
+        const unsigned int f = pack_fold((unsigned int)key & ((1u << shift) - 1u),
+                                         (unsigned int)key >> shift);
+        const unsigned int c1 = bucket1((int)f, lgb), c2 = bucket2((int)f, lgb);
+        for (unsigned int q = 0; q < 4; q++) {
+            const int prev = atomicCAS(tab + 2 * (q < 2 ? c1 : c2) + (q & 1u), kEmpty, key);
+            if (prev == kEmpty || prev == key)
+                return false;
+        }
+        const unsigned int slot = 2 * ((it & 1) ? c2 : c1) + (((unsigned int)it >> 1) & 1u);
+        key = atomicExch(tab + slot, key);
+        if (key == kEmpty)
+            return false;
     }
+    return true;
+}
+
+// The row (lane index of the pack's rows) that holds each of the first
+// `total` <= 64 entries; incl / d: a row's inclusive entry count and length.
+__device__ __forceinline__ int pack_rows_of(int incl, int d, int n, int *mark)
+{
+    const int lane = lane_id();
+    if (lane < n && d > 0)
+        mark[incl - d] = lane;
+    wave_sync();
+    const int m = mark[lane];
+    mark[lane] = 0;
+    wave_sync();
+    return wave_scan_max(m);
+}
+
+// Probes a pack's lists; `row`: this lane's entry's row.  Returns the
+// wave's hits (gather mode: its checksum).
+template <typename OffT, int kMode>
+__device__ __forceinline__ unsigned long long probe_pack(const Group<OffT> &g, int row,
+                                                         const int32_t *__restrict__ adjP,
+                                                         const int *tab, int lg, int shift, int *mark)
+{
+    constexpr int kU = kUnroll;
+    const int lane = lane_id();
+    const int lgb = lg - 1;
+    int carry = 0;  // list of the last position before the window
+    unsigned long long total = 0;
+    unsigned int checksum = 0;
+    // ids of the windows at [at, at + kU * 64) and the rows they are probed for
+    auto fetch = [&](int at, int (&w)[kU], int (&r)[kU]) {
+        OffT idx[kU];
+#pragma unroll
+        for (int k = 0; k < kU; k++) {
+            const int bk = at + k * kWave;
+            idx[k] = 0;
+            r[k] = 0;
+            if (bk < g.total) {
+                const unsigned int off = (unsigned int)(g.excl - bk);
+                if (g.deg > 0 && off < (unsigned int)kWave)
+                    mark[off] = lane;
+                wave_sync();
+                const int m = mark[lane];
+                mark[lane] = 0;
+                wave_sync();
+                const int j = max(wave_scan_max(m), carry);
+                carry = readlane(j, 63);
+                const OffT b = shfl_idx(g.base, j);  // with every lane active
+                r[k] = shfl_idx(row, j);
+                // positions past the end read adjP[0], which exists
+                idx[k] = bk + lane < g.total ? b + (OffT)(bk + lane) : (OffT)0;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kU; k++)
+            w[k] = adjP[idx[k]];
+    };
+    auto lookup = [&](int at, const int (&w)[kU], const int (&r)[kU]) {
+        if constexpr (kMode == kModeGather) {
+#pragma unroll
+            for (int k = 0; k < kU; k++)
+                checksum += at + k * kWave + lane < g.total ? (unsigned int)w[k] : 0u;
+        } else {
+            int2 x1[kU], x2[kU];
+            int key[kU];
+#pragma unroll
+            for (int k = 0; k < kU; k++) {
+                const unsigned int f = pack_fold((unsigned int)w[k], (unsigned int)r[k]);
+                key[k] = at + k * kWave + lane < g.total ? w[k] | r[k] << shift : kNoProbe;
+                x1[k] = bucket_load<false>(tab, bucket1((int)f, lgb));
+                x2[k] = bucket_load<false>(tab, bucket2((int)f, lgb));
+            }
+#pragma unroll
+            for (int k = 0; k < kU; k++) {
+                const unsigned long long m = __builtin_amdgcn_ballot_w64(x1[k].x == key[k]) |
+                                             __builtin_amdgcn_ballot_w64(x1[k].y == key[k]) |
+                                             __builtin_amdgcn_ballot_w64(x2[k].x == key[k]) |
+                                             __builtin_amdgcn_ballot_w64(x2[k].y == key[k]);
+                total += (unsigned int)__popcll(m);
+            }
+        }
+    };
+    int w[kU], r[kU];
+    fetch(0, w, r);
+    for (int at = 0;;) {
+        const int next = at + kU * kWave;
+        if (next >= g.total) {
+            lookup(at, w, r);
+            break;
+        }
+        int wn[kU], rn[kU];
+        fetch(next, wn, rn);
+        lookup(at, w, r);
+#pragma unroll
+        for (int k = 0; k < kU; k++) {
+            w[k] = wn[k];
+            r[k] = rn[k];
+        }
+        at = next;
+    }
+    if constexpr (kMode == kModeGather)
+        total += wave_sum((unsigned long long)checksum);
+    return total;
+}
+
+// Counts the vertices at list positions [i, ...) that fit one pack, at least
+// one and none at or past `last`; returns how many.
+template <typename OffT, int kMode, int kU>
+__device__ __forceinline__ int wave_next(ArgP<OffT> a, long long i, long long last, int *tab,
+                                         int *mark, unsigned long long *sum)
+{
+    constexpr bool kTable = kMode != kModeGather;
+    const int lane = lane_id();
+    const bool in = i + lane < last;
+    const int u = in ? a->list[i + lane] : 0;
+    OffT sH = 0, sW = 0;
+    int dH = 0, dW = 0;
+    const bool same = a->begH == a->begW && a->adjH == a->adjW;
+    if (in) {
+        sH = a->begH[u];
+        dH = (int)(a->begH[u + 1] - sH);
+        if (same) {
+            sW = sH;
+            dW = dH;
+        } else {
+            sW = a->begW[u];
+            dW = (int)(a->endW[u] - sW);
+        }
+    }
+    const int u0 = readlane(u, 0);
+    if constexpr (kMode == kModeBatch)
+        graph_enter(a, mark + kWave, u0);
+    if constexpr (kMode != kModeInstr) {
+        const int iH = wave_scan_add(min(dH, kWave + 1));
+        const int iW = same ? iH : wave_scan_add(min(dW, kWave + 1));
+        bool fits = in && lane < a->pack_rows && iH <= kWave && iW <= kWave;
+        if constexpr (kMode == kModeBatch) {  // one graph
+            const int2 range = *(const int2 *)(mark + kWave);
+            fits = fits && u >= range.x && u < range.y;
+        }
+        const unsigned long long out = ~__ballot(fits);
+        const int n = out ? __builtin_ctzll(out) : kWave;
+        if (n > 1) {
+            const int shift = a->tag_shift;
+            const int lg = min(kPackLg, a->wave_lg);
+            int row = pack_rows_of(iH, dH, n, mark);
+            const int keys = readlane(iH, n - 1);
+            int id = 0;
+            bool failed = false;
+            if (kTable || same) {
+                const OffT at = shfl_idx((OffT)(sH - (OffT)(iH - dH)), row) + (OffT)lane;
+                id = lane < keys ? a->adjH[at] : 0;
+            }
+            if constexpr (kTable) {
+                for (int k = lane; k < 1 << lg; k += kWave)
+                    tab[k] = kEmpty;
+                wave_sync();
+                if (lane < keys)
+                    failed = pack_insert(tab, lg - 1, id | row << shift, shift);
+                wave_sync();
+            }
+            if (__ballot(failed) == 0) {
+                int entries = keys;
+                OffT at = 0;
+                if (!same || a->entW) {
+                    if (!same) {
+                        row = pack_rows_of(iW, dW, n, mark);
+                        entries = readlane(iW, n - 1);
+                    }
+                    at = shfl_idx((OffT)(sW - (OffT)(iW - dW)), row) + (OffT)lane;
+                }
+                const bool valid = lane < entries;
+                const Group<OffT> g = !same || a->entW ? walk_group(a, at, valid)
+                                                       : load_group(id, valid, a->begP);
+                unsigned long long hits = 0;
+                if (g.total > 0)
+                    hits = probe_pack<OffT, kMode>(g, row, a->adjP, tab, lg, shift, mark);
+                wave_sync();
+                add_result<kMode>(sum, mark, hits, (unsigned long long)g.total);
+                return n;
+            }
+        }
+    }
+    wave_vertex<OffT, kMode, kU>(a, u0, readlane(sH, 0), readlane(dH, 0), readlane(sW, 0),
+                                 readlane(dW, 0), tab, mark, sum);
+    return 1;
+}
+
+// ------------------------------------------------------------ the kernel
+// Chunks of `chunk` list positions that belong to this rank (chunk c is rank
+// c % nranks's), out of a tier of `items` (< 2^31) positions.
+__device__ __forceinline__ unsigned int rank_chunks(long long items, int chunk, int rank, int nranks)
+{
+    const unsigned int n = ((unsigned int)items + (unsigned int)chunk - 1u) / (unsigned int)chunk;
+    if (nranks == 1)
+        return n;
+    return n > (unsigned int)rank
+               ? (n - (unsigned int)rank + (unsigned int)nranks - 1u) / (unsigned int)nranks
+               : 0u;
+}
+
+// A queue of n chunks over S counters (kShardStride apart).  Shard s hands
+// out chunks s, s + S, ... (the list order is kept across shards), or with
+// kContig the s-th contiguous part.  From S workgroups on every shard is the
+// home of some of them (blockIdx % S).  A wave leaves its home only when that
+// is empty, so a shard's last chunks are always taken; it then helps the next
+// three shards, which level interleaved ones, and no more: looking for
+// leftovers in all of them, 8192 waves took 94 us to find them empty at the
+// end of every count.  Parts of unequal work, and shards that may have no
+// home, are all tried.  All 64 lanes call; returns n when nothing is left.
+constexpr unsigned int kShardTries = 4;
+template <int S, bool kContig>
+__device__ __forceinline__ unsigned int queue_take(unsigned int *next, unsigned int n,
+                                                   unsigned int &shard, unsigned int groups)
+{
+    static_assert((S & (S - 1)) == 0, "a power of two");
+    const unsigned int per = (n + S - 1) / S;
+    auto share = [&](unsigned int s) -> unsigned int {  // chunks of shard s
+        if constexpr (kContig)
+            return s * per < n ? min(per, n - s * per) : 0u;
+        else
+            return (n + S - 1u - s) / S;
+    };
+    const unsigned int tries = kContig || groups < S ? S : kShardTries;
+    for (unsigned int dry = 0;;) {
+        unsigned int k = 0;
+        if (lane_id() == 0)
+            k = atomicAdd(next + shard * kShardStride, 1u);
+        k = __builtin_amdgcn_readfirstlane(k);
+        if (k < share(shard))
+            return kContig ? shard * per + k : k * S + shard;
+        if (++dry >= tries)
+            return n;
+        shard = (shard + 1) & (S - 1);
+    }
+}
+
+// No more chunks than workgroups: workgroup b counts chunk b, no counter is
+// touched.  The queue's bounds are read again for each chunk: held in scalar
+// registers they would be live across the probe walk.
+constexpr unsigned int kFixed = ~0u;
+template <typename OffT, int kMode, bool kGlobal, int kU>
+__device__ __forceinline__ void group_phase(int tier, unsigned int groups,
+                                            int *tab, int cap_lg, int *mark, int *misc, int *ctot)
+{
+    unsigned int shard = blockIdx.x % kGroupShards;
+    do {
+        ArgP<OffT> a = args_again<OffT>();
+        const long long lb = a->ctl->list_begin[tier], le = a->ctl->list_begin[tier + 1];
+        const unsigned int n = rank_chunks(le - lb, a->chunk_group, a->rank, a->nranks);
+        unsigned int k = blockIdx.x;
+        if (n <= groups) {
+            shard = kFixed;
+        } else {
+            __syncthreads();
+            if (__builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave) == 0)
+                misc[1] = (int)queue_take<kGroupShards, false>(a->ctl->group_next[tier], n, shard,
+                                                               groups);
+            __syncthreads();
+            k = (unsigned int)__builtin_amdgcn_readfirstlane(misc[1]);
+        }
+        if (k >= n)
+            break;
+        const long long first = lb + ((long long)k * a->nranks + a->rank) * a->chunk_group;
+        const long long last = min(first + (long long)a->chunk_group, le);
+        for (long long i = first; i < last; i++)
+            group_vertex<OffT, kGlobal, kMode, kU>(args_again<OffT>()->list[i], tab, cap_lg, mark,
+                                                   misc, ctot);
+    } while (shard != kFixed);
 }
 
 // Waves per SIMD: with int32 offsets eight, and the compiler fits the
@@ -750,88 +1068,83 @@ constexpr int kMinWavesPerEU = sizeof(OffT) == 4 ? 8 : 7;
 
 template <typename OffT, int kMode, bool kBig, int kU = kUnroll>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(kMinWavesPerEU<OffT>, 8)))
-tc_count_kernel(TcArgs<OffT> a)
+tc_count_kernel(TcArgs<OffT>)
 {
+    ArgP<OffT> a = args_again<OffT>();
     extern __shared__ int lds[];
     const int nwaves = blockDim.x / kWave;
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);  // uniform
     const int lane = lane_id();
-    int *mark = lds + a.table_words + wave * kMarkStride;  // + the graph state (batch mode)
-    int *misc = lds + a.table_words + nwaves * kMarkStride;  // 8 words
+    int *mark = lds + a->table_words + wave * kMarkStride;  // + the graph state (batch mode)
+    int *misc = lds + a->table_words + nwaves * kMarkStride;  // 8 words, the last four: sums
     int *ctot = misc + 8;                                     // kMaxChunks + 1 words
+    unsigned long long *sum = (unsigned long long *)(misc + 4);  // triangles, probes
     mark[lane] = 0;
-    unsigned long long acc = 0, probes = 0;
+    if (wave == 0 && lane < 2)
+        sum[lane] = 0;
+    __syncthreads();
     if constexpr (kMode == kModeBatch) {
         graph_init(mark + kWave);
-        if (threadIdx.x == 0)
-            atomicMin(a.graph_t0, (unsigned long long)wall_clock64());
+        if (wave == 0 && lane == 0)
+            atomicMin(a->graph_t0, (unsigned long long)wall_clock64());
     }
 
-    if (kBig && a.spill_tier >= 0 && (int)blockIdx.x < a.spill_groups) {
-        int *tab = a.spill_mem + (long long)blockIdx.x * a.spill_slots;
+    if (kBig && a->spill_tier >= 0 && (int)blockIdx.x < a->spill_groups) {
+        int *tab = a->spill_mem + (long long)blockIdx.x * a->spill_slots;
         int cap_lg = 0;
-        while ((2ll << cap_lg) <= a.spill_slots)
+        while ((2ll << cap_lg) <= a->spill_slots)
             cap_lg++;
-        group_phase<OffT, kMode, true, kU>(a, a.spill_tier, tab, cap_lg, mark, misc, ctot, acc, probes);
+        group_phase<OffT, kMode, true, kU>(a->spill_tier, (unsigned int)a->spill_groups, tab, cap_lg,
+                                           mark, misc, ctot);
     }
-    if (a.group_tier >= 0)
-        group_phase<OffT, kMode, false, kU>(a, a.group_tier, lds, a.group_lg, mark, misc, ctot, acc,
-                                        probes);
+    if (a->group_tier >= 0)
+        group_phase<OffT, kMode, false, kU>(a->group_tier, gridDim.x, lds, a->group_lg, mark, misc,
+                                            ctot);
     __syncthreads();  // the wave tables reuse the group table's LDS
-    if (!kBig && a.wave_tier >= 0) {
-        const long long lb = a.ctl->list_begin[a.wave_tier];
-        const long long le = a.ctl->list_begin[a.wave_tier + 1];
-        int *wtab = lds + wave * a.wave_slots;
-        // Shard s hands out the rank's chunks j with j % kQueueShards == s
-        // (chunk c = j * nranks + rank, the reference's interleave), so the
-        // list order is kept across shards.  A wave starts on shard
-        // blockIdx % kQueueShards and moves on when a shard runs dry; after
-        // finding every shard dry once it is done.
+    if (!kBig && a->wave_tier >= 0) {
+        int *wtab = lds + wave * a->wave_slots;
+        // Chunk j of the rank is chunk j * nranks + rank of the list, the
+        // reference's interleave.  A single large graph interleaves the
+        // shards, which spreads each vertex range over all eight L2s (R-MAT
+        // 26: contiguous shards measured up to 3% slower).  A batch's list
+        // is in graph order: its shards are contiguous eighths, one for the
+        // workgroups of each XCD (dealt round-robin), so the graphs that an
+        // XCD counts at a time stay in its L2 (10k-graph ER/BA batch: 4.8%
+        // faster; four parts per XCD measured 17% slower than one).
         //
-        // Batches instead give shard s the s-th contiguous eighth of the
-        // rank's chunks and start a wave on the shard of its XCD: the list
-        // is in graph order, so each XCD counts its own graphs and their
-        // lists stay in its L2 (10k-graph ER/BA batch: 4.8% faster).  A
-        // single large graph keeps the interleave, which spreads each
-        // vertex range over all eight L2s (R-MAT 26: contiguous shards
-        // measured up to 3% slower).
-        constexpr bool kContig = kMode == kModeBatch;
-        int shard = kContig ? xcc_id() : (int)(blockIdx.x % kQueueShards);
-        long long per = 0;  // chunks per contiguous shard
-        if constexpr (kContig) {
-            const long long nchunk = (le - lb + a.chunk_wave - 1) / a.chunk_wave;
-            const long long nmine = nchunk > a.rank ? (nchunk - a.rank + a.nranks - 1) / a.nranks : 0;
-            per = (nmine + kQueueShards - 1) / kQueueShards;
-        }
-        int dry = 0;
-        while (dry < kQueueShards) {
-            unsigned int k = 0;
-            if (lane == 0)
-                k = atomicAdd(&a.ctl->shard[shard * kShardStride], 1u);
-            k = __builtin_amdgcn_readfirstlane(k);
-            const long long j = kContig ? (long long)shard * per + (long long)k
-                                        : (long long)k * kQueueShards + shard;
-            const long long first = lb + (j * a.nranks + a.rank) * a.chunk_wave;
-            if ((kContig && (long long)k >= per) || first >= le) {
-                dry++;
-                shard = shard + 1 == kQueueShards ? 0 : shard + 1;
-                continue;
-            }
-            const long long last = min(first + (long long)a.chunk_wave, le);
-            for (long long i = first; i < last; i++)
-                wave_vertex<OffT, kMode, kU>(a, a.list[i], wtab, mark, acc, probes);
-        }
+        // With no more chunks than waves, wave w takes chunk w and no
+        // counter is touched; consecutive chunks go to different workgroups
+        // (the list's first chunks are its heaviest).
+        const long long items = a->ctl->list_begin[kTierWave + 1] - a->ctl->list_begin[kTierWave];
+        // chosen here: at least two grabs per wave, at most 64 vertices each
+        // (larger chunks of a skewed list leave long ones for the end)
+        int chunk = a->chunk_wave;
+        if (chunk <= 0)
+            chunk = max(1, min(kWave, (int)(items / (2ll * gridDim.x * nwaves))));
+        const unsigned int n = rank_chunks(items, chunk, a->rank, a->nranks);
+        constexpr bool kBatch = kMode == kModeBatch;
+        constexpr int kShards = kBatch ? kXcds : kWaveShards;
+        const bool fixed = !kBatch && n <= gridDim.x * (unsigned int)nwaves;
+        unsigned int shard = kBatch ? (unsigned int)xcc_id() : blockIdx.x % kShards;
+        do {
+            const unsigned int j = fixed ? (unsigned int)wave * gridDim.x + blockIdx.x
+                                         : queue_take<kShards, kBatch>(a->ctl->wave_next, n, shard,
+                                                                       gridDim.x);
+            if (j >= n)
+                break;
+            const long long lb = a->ctl->list_begin[kTierWave], le = a->ctl->list_begin[kTierWave + 1];
+            const long long first = lb + ((long long)j * a->nranks + a->rank) * chunk;
+            const long long last = min(first + (long long)chunk, le);
+            for (long long i = first; i < last;)
+                i += wave_next<OffT, kMode, kU>(a, i, last, wtab, mark, sum);
+        } while (!fixed);
     }
     if constexpr (kMode == kModeBatch)
-        graph_flush(a, mark + kWave, acc);  // acc is now 0: the batch total is the graphs' sum
-    acc = wave_sum(acc);
-    probes = wave_sum(probes) / kWave;  // every lane carried the wave's probe total
-    if (lane == 0) {
-        if (acc)
-            atomicAdd(&a.ctl->count, acc);
-        if (probes)
-            atomicAdd(&a.ctl->probes, probes);
-    }
+        graph_flush(a, mark + kWave);  // the batch total is the graphs' sum
+    // one pair of atomics per workgroup
+    __syncthreads();
+    if (wave == 0 && lane < 2 && sum[lane] && (kMode != kModeBatch || lane == 1))
+        atomicAdd(&a->ctl->sums[blockIdx.x % kSumLines].count + lane, sum[lane]);
 }
 
 // ------------------------------------------------------------- planning

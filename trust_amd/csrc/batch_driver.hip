@@ -144,7 +144,7 @@ int enqueue_segments(Ctx *ctx, const trust_params &p, int mode, const ResidentRu
 {
     const DevCsr &g = ctx->g;
     const int64_t ng = ctx->batch_ngraphs;
-    int rc = ctx->list.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(g.V, 1));
+    int rc = ctx->list.ensure(sizeof(int32_t) * (size_t)(g.V + kMaxExtra));
     if (rc)
         return rc;
     unsigned long long *out = (unsigned long long *)ctx->batch_out.p;
@@ -199,6 +199,8 @@ int read_ctl(Ctx *ctx, const ResidentRun &R, TcCtl &h)
         h.rebuilds += hs[k].rebuilds;
         for (int t = 0; t < 8; t++)
             h.list_begin[t] += hs[k].list_begin[t];
+        for (int t = 0; t < 8; t++)
+            h.extra[t] += hs[k].extra[t];
     }
     return TRUST_OK;
 }

@@ -53,6 +53,7 @@ struct CsrViews {
     const void *entW = nullptr;
     // ids of the hash and probe rows are below this
     int64_t ids = int64_t(1) << 31;
+    int64_t entries = 0;  // of the walk rows (0: not known; an upper bound will do)
 };
 
 // Shape of one counting launch.

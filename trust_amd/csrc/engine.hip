@@ -272,21 +272,22 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
                   bool preplanned, hipStream_t s, hipEvent_t ev_plan, hipEvent_t ev_count,
                   const SegView *seg, bool plan_only, bool with_core)
 {
-    int rc = ctx->list.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(V, 1));
+    int rc = ctx->list.ensure(sizeof(int32_t) * (size_t)(V + kMaxExtra));
     if (rc)
         return rc;
-    const int per_block = kPlanPerBlock;
-    const int nblocks = (int)((V + per_block - 1) / per_block);
-    rc = ctx->block_counts.ensure(sizeof(long long) * (size_t)kNumTiers * std::max(nblocks, 1));
+    rc = ctx->block_counts.ensure(kPlanScratch);
     if (rc)
         return rc;
+    // a list made elsewhere, and the instrumented mode's per-vertex outputs,
+    // know whole vertices only
+    const int part_entries =
+        preplanned || seg || (mode & ~kProbeDeep) == kModeInstr ? 0 : walk_part_entries(views.entries);
     if (L.spill_groups > 0) {
         rc = ctx->spill.ensure(sizeof(int32_t) * (size_t)L.spill_slots * L.spill_groups);
         if (rc)
             return rc;
     }
     if (!preplanned) {
-        HIPCHK(launch_fill_u32((uint32_t *)ctl_dev, 0u, sizeof(TcCtl) / 4, s));
         PlanArgs<OffT> pa;
         memset(&pa, 0, sizeof(pa));
         pa.begH = (const OffT *)views.begH;
@@ -300,12 +301,11 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
         pa.big_lg = L.has_big ? L.big.group_lg : 0;
         pa.force_spill = (p.flags & TRUST_FLAG_FORCE_SPILL) ? 1 : 0;
         pa.wave_only = (p.flags & TRUST_FLAG_WAVE_ONLY) ? 1 : 0;
-        pa.tier_override = nullptr;
+        pa.part_entries = part_entries;
         pa.list = seg ? (int32_t *)seg->list : (int32_t *)ctx->list.p;
-        pa.block_counts = (long long *)ctx->block_counts.p;
-        pa.per_block = per_block;
+        pa.block_counts = (int *)ctx->block_counts.p;
         pa.ctl = ctl_dev;
-        HIPCHK(launch_plan<OffT>(pa, nblocks, s));
+        HIPCHK(launch_plan<OffT>(pa, s));
     }
     if (ev_plan)
         HIPCHK(hipEventRecord(ev_plan, s));
@@ -331,6 +331,7 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
     TcArgs<OffT> a;
     if (L.has_big) {
         fill_args(a, ctx, views, p, L, L.big, ctl_dev, instr_cycles, instr_probes, seg);
+        a.part_entries = part_entries;
         a.spill_tier = L.spill_groups > 0 ? kTierSpill : -1;
         a.group_tier = kTierBig;
         a.wave_tier = -1;
@@ -345,6 +346,7 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
             HIPCHK(hipEventRecord(ctx->ev_join, ctx->aux_stream));
     }
     fill_args(a, ctx, views, p, L, L.main, ctl_dev, instr_cycles, instr_probes, seg);
+    a.part_entries = part_entries;
     a.spill_tier = -1;
     a.group_tier = kTierHub;
     a.wave_tier = kTierWave;
@@ -755,6 +757,7 @@ int enqueue_resident(Ctx *ctx, const trust_params &p, int mode, const ResidentRu
     CsrViews v{g.beg.p, (const int32_t *)g.adj.p, g.beg.p, (const int32_t *)g.adj.p, g.beg.p,
                (const int32_t *)g.adj.p};
     v.ids = g.V;
+    v.entries = g.E;  // the short-side walk's rows hold fewer
     if (timed)
         HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
     int rc;
@@ -762,6 +765,8 @@ int enqueue_resident(Ctx *ctx, const trust_params &p, int mode, const ResidentRu
         v.begW = ctx->side_beg.p;
         v.adjW = nullptr;
         v.entW = ctx->side_ent.p;
+        if (ctx->side_entries >= 0)
+            v.entries = ctx->side_entries;
     } else if (R.starts) {  // walk rows = N+, each entry's list read from the start index
         v.entW = ctx->ref_ent.p;
     }
@@ -823,7 +828,7 @@ int finish_resident(Ctx *ctx, ResidentRun &R, const TcCtl &h, double t_plan, dou
                  : R.starts ? alg_bytes_starts(g.V, g.E, h.probes, g.off64 && !R.segmented)
                           : alg_bytes(g.V, g.E, h.probes, g.off64 && !R.segmented);
     r->n_spill = h.list_begin[kTierSpill + 1] - h.list_begin[kTierSpill];
-    r->n_hub = h.list_begin[kTierHub + 1] - h.list_begin[kTierBig];  // big + hub
+    r->n_hub = group_vertices(h);  // big + hub
     r->n_wave = h.list_begin[kTierWave + 1] - h.list_begin[kTierWave];
     r->threads = L.main.threads;
     r->blocks = L.main.blocks;

@@ -27,13 +27,11 @@ namespace trust {
 constexpr int64_t kNoAllocMaxV = int64_t(1) << 22;
 constexpr size_t kScrCtl = 0;                      // TcCtl
 constexpr size_t kScrMisc = 16384;                 // NoAllocMisc
-constexpr size_t kScrBlocks = 20480;               // kNumTiers x planner blocks (long long)
-constexpr size_t kScrBlocksBytes = sizeof(long long) * kNumTiers *
-                                   ((kNoAllocMaxV + kPlanPerBlock - 1) / kPlanPerBlock);
+constexpr size_t kScrBlocks = 20480;               // the planner's counts
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
-constexpr size_t kScrBeg = align256(kScrBlocks + kScrBlocksBytes);       // int32 offsets
+constexpr size_t kScrBeg = align256(kScrBlocks + kPlanScratch);          // int32 offsets
 constexpr size_t kScrList = align256(kScrBeg + 4 * (kNoAllocMaxV + 1));  // tier list
-constexpr size_t kScratchBytes = align256(kScrList + 4 * kNoAllocMaxV);
+constexpr size_t kScratchBytes = align256(kScrList + 4 * (kNoAllocMaxV + kMaxExtra));
 static_assert(sizeof(TcCtl) <= kScrMisc - kScrCtl, "control block does not fit");
 
 struct NoAllocMisc {
@@ -145,7 +143,7 @@ extern "C" int trust_count_csr_noalloc(const int64_t *beg_dev, const int32_t *ad
     hipStream_t s = (hipStream_t)stream;
     TcCtl *ctl = (TcCtl *)(scr + kScrCtl);
     NoAllocMisc *misc = (NoAllocMisc *)(scr + kScrMisc);
-    long long *block_counts = (long long *)(scr + kScrBlocks);
+    int *block_counts = (int *)(scr + kScrBlocks);
     int32_t *beg32 = (int32_t *)(scr + kScrBeg);
     int32_t *list = (int32_t *)(scr + kScrList);
 
@@ -192,7 +190,6 @@ extern "C" int trust_count_csr_noalloc(const int64_t *beg_dev, const int32_t *ad
                     "does not have", hm.max_deg);
 
     hipLaunchKernelGGL(na_stamp_kernel, dim3(1), dim3(1), 0, s, &misc->t0);
-    const int nblocks = (int)((V + kPlanPerBlock - 1) / kPlanPerBlock);
     PlanArgs<int32_t> pa;
     memset(&pa, 0, sizeof(pa));
     pa.begH = pa.begW = beg32;
@@ -206,15 +203,16 @@ extern "C" int trust_count_csr_noalloc(const int64_t *beg_dev, const int32_t *ad
     pa.wave_only = (p->flags & TRUST_FLAG_WAVE_ONLY) ? 1 : 0;
     pa.list = list;
     pa.block_counts = block_counts;
-    pa.per_block = kPlanPerBlock;
+    pa.part_entries = walk_part_entries(E);
     pa.ctl = ctl;
-    HIPCHK(launch_plan<int32_t>(pa, nblocks, s));
+    HIPCHK(launch_plan<int32_t>(pa, s));
     TcArgs<int32_t> a;
     memset(&a, 0, sizeof(a));
     a.begH = a.begW = a.begP = beg32;
     a.endW = beg32 + 1;
     a.adjH = a.adjW = a.adjP = adj_dev;
     a.list = list;
+    a.part_entries = walk_part_entries(E);
     a.spill_tier = -1;
     a.chunk_group = L.chunk_group;
     a.chunk_wave = L.chunk_wave;
@@ -263,7 +261,7 @@ extern "C" int trust_count_csr_noalloc(const int64_t *beg_dev, const int32_t *ad
         r->gteps = r->seconds > 0 ? (double)E / r->seconds / 1e9 : 0.0;
         r->alg_bytes = alg_bytes(V, E, h.probes, false);
         r->n_spill = 0;
-        r->n_hub = h.list_begin[kTierHub + 1] - h.list_begin[kTierBig];
+        r->n_hub = group_vertices(h);
         r->n_wave = h.list_begin[kTierWave + 1] - h.list_begin[kTierWave];
         r->threads = L.main.threads;
         r->blocks = L.main.blocks;

@@ -303,10 +303,9 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
     const size_t stage_bytes = ((sizeof(int32_t) * (size_t)maxE + 255) & ~(size_t)255) +
                                sizeof(int64_t) * (size_t)(maxV + 1);
     const bool pinned_uploads = stage.init(stage_bytes);
-    rc = ctx->list.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(maxV, 1));
+    rc = ctx->list.ensure(sizeof(int32_t) * (size_t)(maxV + kMaxExtra));
     if (!rc)
-        rc = ctx->block_counts.ensure(sizeof(long long) * kNumTiers *
-                                      (size_t)std::max<int64_t>((maxV + kPlanPerBlock - 1) / kPlanPerBlock, 1));
+        rc = ctx->block_counts.ensure(kPlanScratch);
     if (rc)
         return rc;
     struct SlotGuard {
@@ -540,16 +539,19 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
             const TileWalk &w = walks[(size_t)jk];
             CsrViews vo{th.beg.p, (const int32_t *)th.adj.p, w.out_beg.p,
                         (const int32_t *)w.out_ids.p, tp.beg.p, (const int32_t *)tp.adj.p};
+            vo.entries = w.x_out;
             if ((rc = count_view(vo, rows_of[ji], (TcCtl *)ctls.p + 2 * job)))
                 return rc;
             CsrViews vi{tp.beg.p, (const int32_t *)tp.adj.p, w.in_beg.p,
                         (const int32_t *)w.in_ids.p, th.beg.p, (const int32_t *)th.adj.p};
+            vi.entries = w.x_in;
             if ((rc = count_view(vi, rows_of[jk], (TcCtl *)ctls.p + 2 * job + 1)))
                 return rc;
         } else {
             const DevCsr &tw = slots[sl[1]].g;
             CsrViews v{th.beg.p, (const int32_t *)th.adj.p, tw.beg.p, (const int32_t *)tw.adj.p,
                        tp.beg.p, (const int32_t *)tp.adj.p};
+            v.entries = tw.E;
             if ((rc = count_view(v, tiles[cur[0]].vertices, (TcCtl *)ctls.p + job)))
                 return rc;
         }
@@ -777,6 +779,7 @@ extern "C" int trust_triangle_count_partition(int rank, const char *folder, int 
         return rc;
     CsrViews v{d[0].beg.p, (const int32_t *)d[0].adj.p, d[1].beg.p, (const int32_t *)d[1].adj.p,
                d[2].beg.p, (const int32_t *)d[2].adj.p};
+    v.entries = t[1].edges;
     HIPCHK(hipEventRecord(ctx.ev[0], ctx.stream));
     rc = off64 ? enqueue_count<int64_t>(&ctx, v, t[0].vertices, false, p, L, (TcCtl *)ctx.ctl.p,
                                         kModeCount, nullptr, nullptr, false, ctx.stream, ctx.ev[1],

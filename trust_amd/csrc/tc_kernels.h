@@ -17,7 +17,7 @@ enum Tier : int { kTierSpill = 0, kTierBig = 1, kTierHub = 2, kTierWave = 3, kTi
 constexpr int kNumTiers = 4;
 constexpr int kWave = 64;
 constexpr int kMinTableLg = 6;       // smallest table: 64 slots
-constexpr int kPlanPerBlock = 4096;  // vertices per planning workgroup
+constexpr int kPlanBlocks = 2048;    // planning workgroups, at most
 constexpr int kMaxChunks = 256;      // 64-neighbour chunks balanced per group vertex
 // Probe windows in flight per wave (the probe walk's batch): four, or six
 // with kProbeDeep.  Six keep more loads in flight where the probed lists are
@@ -63,6 +63,7 @@ struct alignas(128) TcCtl {
     unsigned long long count;       // triangles       (totals: host side,
     unsigned long long probes;      // hash lookups (W) fold_ctl)
     long long list_begin[8];        // tier t occupies list[list_begin[t], list_begin[t+1])
+    int extra[8];                   // of them, positions beyond a vertex's first (group_parts)
     unsigned long long rebuilds;    // tables rebuilt with linear probing after a cuckoo attempt
     TcSum sums[kSumLines];          // triangles and hash lookups, by workgroup
     // queue cursors (a copy to the host needs none of what follows: kCtlHead)
@@ -71,6 +72,11 @@ struct alignas(128) TcCtl {
 };
 // Bytes of a control block that hold results (list bounds, sums).
 constexpr size_t kCtlHead = offsetof(TcCtl, wave_next);
+// Vertices of the workgroup tiers with LDS tables (big and hub).
+inline long long group_vertices(const TcCtl &h)
+{
+    return h.list_begin[kTierHub + 1] - h.list_begin[kTierBig] - h.extra[kTierBig] - h.extra[kTierHub];
+}
 // Totals of a control block copied back to the host.
 inline void fold_ctl(TcCtl &h)
 {
@@ -114,6 +120,7 @@ struct TcArgs {
     int wave_lg;
     int chunk_group;         // vertices per grab, spill/group tiers
     int chunk_wave;          // vertices per grab, wave tier (0: chosen by the kernel)
+    int part_entries;        // walk entries of a workgroup-tier part (0: vertices are whole)
     int pack_rows;           // rows a pack of the wave tier may hold (0, 1: no packs)
     int tag_shift;           // bits of an id (a pack's keys are id | row << tag_shift)
     int rank;
@@ -151,16 +158,18 @@ struct PlanArgs {
     int big_lg;         // log2 of the large-LDS launch's table (0: no such launch)
     int force_spill;
     int wave_only;
-    const unsigned char *tier_override;  // nullable: per-vertex tier chosen elsewhere
-    int32_t *list;
-    long long *block_counts;  // [kNumTiers][nblocks]
-    int per_block;
+    int part_entries;   // see group_parts (0: vertices stay whole)
+    int32_t *list;      // V + kMaxExtra positions
+    int *block_counts;  // kPlanBlocks x 2 kNumTiers
+    int per_block;      // set by launch_plan
     TcCtl *ctl;
 };
 
+constexpr size_t kPlanScratch = sizeof(int) * 2 * kNumTiers * kPlanBlocks;  // PlanArgs::block_counts
+
 // Launch wrappers (tc_kernels.hip).  All launches go on `stream`.
 template <typename OffT>
-hipError_t launch_plan(const PlanArgs<OffT> &p, int nblocks, hipStream_t stream);
+hipError_t launch_plan(PlanArgs<OffT> p, hipStream_t stream);
 template <typename OffT>
 // big: the large-LDS launch (spill + big tiers), else the main launch.
 hipError_t launch_count(const TcArgs<OffT> &a, int blocks, int threads, size_t lds_bytes,
@@ -212,6 +221,35 @@ hipError_t launch_side_stats(const OffT *beg, const int32_t *adj, long long V,
 // of the reference walk's probes (its lists are shorter, so a probe costs
 // more; measured break-even near 0.45-0.5 on R-MAT).
 constexpr double kShortWalkShare = 0.45;
+
+// Parts of the workgroup tiers.  One vertex's walk can hold a good share of a
+// graph's probes, and the workgroup that takes it counts on when all others
+// are done (R-MAT 20, 2 G probes by the short-side walk: 3.45 ms with whole
+// vertices, 2.5 ms in parts; R-MAT 24 the same either way).  A vertex of
+// more than part_entries walk entries (four times as many in the large-LDS
+// launch, whose workgroups are four times as large) fills one list position
+// per part, and each part builds the vertex's table for itself.
+// part_entries is 1/16384 of the walk, so that no part outlasts the count's
+// average workgroup and the list holds at most kMaxExtra more positions; at
+// least 128, below which building the table costs more than the part's walk.
+constexpr int kBigPartLg = 2;
+constexpr long long kMaxExtra = 16384;
+inline int walk_part_entries(long long walk_entries)
+{
+    if (walk_entries <= 0)
+        return 0;
+    int lg = 7;
+    while (lg < 28 && (kMaxExtra << lg) < walk_entries)
+        lg++;
+    return 1 << lg;
+}
+__host__ __device__ inline int group_parts(int dW, int part_entries, int tier)
+{
+    if (part_entries <= 0)
+        return 1;
+    const int e = part_entries << (tier == kTierBig ? kBigPartLg : 0);
+    return dW > e ? (dW + e - 1) / e : 1;
+}
 
 // Packs of the wave tier (tc_kernels.hip): ids below `ids` leave the upper
 // bits of a 32-bit key for the row's number; the largest number is left out,

@@ -36,6 +36,8 @@
 //    a uint64 in device memory (TC.cu:586-596).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "tc_kernels.h"
 #include "wave_ops.h"
 
@@ -520,7 +522,7 @@ __device__ __forceinline__ unsigned long long probe_windows(const Group<OffT> &g
 // capacity 2^cap_lg.  misc[0]: unit cursor, misc[2]: window total;
 // ctot: kMaxChunks+1 ints of LDS.
 template <typename OffT, bool kGlobal, int kMode, int kU>
-__device__ __forceinline__ void group_vertex(int u, int *tab, int cap_lg,
+__device__ __forceinline__ void group_vertex(int u, int tier, long long at, int *tab, int cap_lg,
                                              int *mark, int *misc, int *ctot)
 {
     constexpr bool kInstr = kMode == kModeInstr;
@@ -537,8 +539,28 @@ __device__ __forceinline__ void group_vertex(int u, int *tab, int cap_lg,
     const int nwaves = blockDim.x / kWave;
     const OffT sH = a->begH[u];
     const int dH = (int)(a->begH[u + 1] - sH);
-    const OffT sW = a->begW[u];
-    const int dW = (int)(a->endW[u] - sW);
+    OffT sW = a->begW[u];
+    int dW = (int)(a->endW[u] - sW);
+    int part = 0;
+    if constexpr (!kGlobal) {
+        const int parts = group_parts(dW, a->part_entries, tier);
+        if (parts > 1) {
+            // the vertex fills `parts` list positions in a row: this one's
+            // number is the count of those before it
+            const int32_t *list = a->list + at;
+            for (int back = 1; back < parts; back += kWave) {
+                const bool mine = back + lane < parts && back + lane <= at &&
+                                  list[-(back + lane)] == u;
+                const unsigned long long m = __ballot(mine);
+                part += __popcll(m);
+                if (~m)
+                    break;
+            }
+            const int entries = a->part_entries << (tier == kTierBig ? kBigPartLg : 0);
+            sW += (OffT)((long long)part * entries);
+            dW = min(entries, dW - part * entries);
+        }
+    }
     const int lg = table_lg(dH, cap_lg);
     const int size = 1 << lg;
     if constexpr (kTable)
@@ -564,7 +586,7 @@ __device__ __forceinline__ void group_vertex(int u, int *tab, int cap_lg,
         __syncthreads();
         linear = misc[3] != 0;
         if (linear) {  // rebuild this vertex's table with linear probing
-            if (tid == 0 && a->force_linear != 1)
+            if (tid == 0 && a->force_linear != 1 && part == 0)
                 atomicAdd(&a->ctl->rebuilds, 1ull);
             __syncthreads();
             for (int i = tid; i < size; i += blockDim.x)
@@ -1048,8 +1070,8 @@ __device__ __forceinline__ void group_phase(int tier, unsigned int groups,
         const long long first = lb + ((long long)k * a->nranks + a->rank) * a->chunk_group;
         const long long last = min(first + (long long)a->chunk_group, le);
         for (long long i = first; i < last; i++)
-            group_vertex<OffT, kGlobal, kMode, kU>(args_again<OffT>()->list[i], tab, cap_lg, mark,
-                                                   misc, ctot);
+            group_vertex<OffT, kGlobal, kMode, kU>(args_again<OffT>()->list[i], tier, i, tab, cap_lg,
+                                                   mark, misc, ctot);
     } while (shard != kFixed);
 }
 
@@ -1148,13 +1170,18 @@ tc_count_kernel(TcArgs<OffT>)
 }
 
 // ------------------------------------------------------------- planning
+// The degree split in two launches: each workgroup counts the tiers of its
+// per_block vertices, then every workgroup sums the counts of those before it
+// (at most kPlanBlocks, 32 bytes each) and writes its vertices' list
+// positions in order.  The first launch also clears the control block.  With
+// a fill, a count, a one-workgroup scan and a scatter a plan took 45-60 us
+// however small the graph; this takes 10-15.
 template <typename OffT>
-__device__ __forceinline__ int plan_tier(const PlanArgs<OffT> &p, long long u)
+__device__ __forceinline__ int plan_tier(const PlanArgs<OffT> &p, long long u, int &parts)
 {
-    if (p.tier_override)
-        return (int)p.tier_override[u];
     const long long dH = (long long)(p.begH[u + 1] - p.begH[u]);
     const long long dW = (long long)(p.endW[u] - p.begW[u]);
+    parts = 1;
     if (dH == 0 || dW == 0 || (p.same_csr && dH < 2))
         return kTierNone;  // contributes nothing (reference skips d+ < 2, TC.cu:440-441)
     int lg = kMinTableLg;
@@ -1162,112 +1189,146 @@ __device__ __forceinline__ int plan_tier(const PlanArgs<OffT> &p, long long u)
         lg++;
     if (p.force_spill || lg > max(p.hub_lg, p.big_lg))
         return kTierSpill;
-    if (lg > p.hub_lg)
+    if (lg > p.hub_lg) {
+        parts = group_parts((int)dW, p.part_entries, kTierBig);
         return kTierBig;
-    if (!p.wave_only && dW > p.hub_threshold)
+    }
+    if ((!p.wave_only && dW > p.hub_threshold) || lg > p.wave_lg) {
+        parts = group_parts((int)dW, p.part_entries, kTierHub);
         return kTierHub;
-    if (lg > p.wave_lg)
-        return kTierHub;
+    }
     return kTierWave;
 }
 
+__device__ __forceinline__ int wave_total(int x) { return readlane(wave_scan_add(x), kWave - 1); }
+
 template <typename OffT>
-__global__ void __launch_bounds__(256) plan_count_kernel(PlanArgs<OffT> p, int nblocks)
+__global__ void __launch_bounds__(1024) plan_count_kernel(PlanArgs<OffT> p)
 {
-    __shared__ unsigned long long cnt[kNumTiers];
-    if (threadIdx.x < kNumTiers)
+    __shared__ int cnt[2 * kNumTiers];  // list positions, then those beyond one per vertex
+    if (threadIdx.x < 2 * kNumTiers)
         cnt[threadIdx.x] = 0;
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < (int)(sizeof(TcCtl) / 4); i += blockDim.x)
+            ((uint32_t *)p.ctl)[i] = 0;
     __syncthreads();
     const long long lo = (long long)blockIdx.x * p.per_block;
     const long long hi = min(lo + p.per_block, p.V);
-    int local[kNumTiers] = {0, 0, 0, 0};
-    for (long long u = lo + threadIdx.x; u < hi; u += blockDim.x) {
-        int t = plan_tier(p, u);
+    int n[kNumTiers] = {0, 0, 0, 0}, more[kNumTiers] = {0, 0, 0, 0};
+    for (long long u0 = lo; u0 < hi; u0 += blockDim.x) {
+        const long long u = u0 + threadIdx.x;
+        int parts = 1;
+        const int t = u < hi ? plan_tier(p, u, parts) : kTierNone;
+        const bool split = __ballot(parts > 1) != 0;
 #pragma unroll
-        for (int q = 0; q < kNumTiers; q++)
-            local[q] += t == q;
-    }
-    for (int t = 0; t < kNumTiers; t++)
-        if (local[t])
-            atomicAdd(&cnt[t], (unsigned long long)local[t]);
-    __syncthreads();
-    if (threadIdx.x < kNumTiers)
-        p.block_counts[(long long)threadIdx.x * nblocks + blockIdx.x] = (long long)cnt[threadIdx.x];
-}
-
-// One workgroup: exclusive scan of the per-block counts of each tier into
-// global write offsets; records the tier boundaries in ctl->list_begin.
-template <typename OffT>
-__global__ void __launch_bounds__(1024) plan_scan_kernel(PlanArgs<OffT> p, int nblocks)
-{
-    __shared__ long long part[1024];
-    __shared__ long long base;
-    if (threadIdx.x == 0)
-        base = 0;
-    __syncthreads();
-    for (int t = 0; t < kNumTiers; t++) {
-        if (threadIdx.x == 0)
-            p.ctl->list_begin[t] = base;
-        for (int c0 = 0; c0 < nblocks; c0 += blockDim.x) {
-            const int i = c0 + threadIdx.x;
-            long long x = i < nblocks ? p.block_counts[(long long)t * nblocks + i] : 0;
-            part[threadIdx.x] = x;
-            __syncthreads();
-            for (int off = 1; off < (int)blockDim.x; off <<= 1) {
-                long long y = threadIdx.x >= (unsigned)off ? part[threadIdx.x - off] : 0;
-                __syncthreads();
-                part[threadIdx.x] += y;
-                __syncthreads();
-            }
-            const long long incl = part[threadIdx.x];
-            if (i < nblocks)
-                p.block_counts[(long long)t * nblocks + i] = base + incl - x;
-            __syncthreads();
-            if (threadIdx.x == blockDim.x - 1)
-                base += incl;
-            __syncthreads();
+        for (int q = 0; q < kNumTiers; q++) {
+            n[q] += __popcll(__ballot(t == q));
+            if (split)
+                more[q] += wave_total(t == q ? parts - 1 : 0);
         }
     }
-    if (threadIdx.x == 0)
-        p.ctl->list_begin[kNumTiers] = base;
+    if (lane_id() == 0)
+        for (int q = 0; q < kNumTiers; q++) {
+            if (n[q])
+                atomicAdd(&cnt[q], n[q] + more[q]);
+            if (more[q])
+                atomicAdd(&cnt[kNumTiers + q], more[q]);
+        }
+    __syncthreads();
+    if (threadIdx.x < 2 * kNumTiers)
+        p.block_counts[(long long)blockIdx.x * 2 * kNumTiers + threadIdx.x] = cnt[threadIdx.x];
 }
 
 template <typename OffT>
-__global__ void __launch_bounds__(256) plan_scatter_kernel(PlanArgs<OffT> p, int nblocks)
+__global__ void __launch_bounds__(1024) plan_scatter_kernel(PlanArgs<OffT> p, int nblocks)
 {
-    __shared__ int wcount[kNumTiers][4];
-    __shared__ long long run[kNumTiers];
-    const int wave = threadIdx.x / kWave, lane = lane_id();
+    __shared__ int all[2 * kNumTiers], before[kNumTiers];
+    __shared__ int wcount[kNumTiers][1024 / kWave];
+    __shared__ int run[kNumTiers];
+    const int wave = threadIdx.x / kWave, nwaves = blockDim.x / kWave;
+    if (threadIdx.x < 2 * kNumTiers)
+        all[threadIdx.x] = 0;
     if (threadIdx.x < kNumTiers)
-        run[threadIdx.x] = p.block_counts[(long long)threadIdx.x * nblocks + blockIdx.x];
+        before[threadIdx.x] = 0;
+    __syncthreads();
+    {
+        int sum[2 * kNumTiers] = {0}, mine[kNumTiers] = {0};
+        for (int b = threadIdx.x; b < nblocks; b += blockDim.x) {
+            const int4 c = ((const int4 *)p.block_counts)[2 * b];
+            const int4 e = ((const int4 *)p.block_counts)[2 * b + 1];
+            const int v[2 * kNumTiers] = {c.x, c.y, c.z, c.w, e.x, e.y, e.z, e.w};
+#pragma unroll
+            for (int q = 0; q < 2 * kNumTiers; q++) {
+                sum[q] += v[q];
+                if (q < kNumTiers && b < (int)blockIdx.x)
+                    mine[q] += v[q];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 2 * kNumTiers; q++) {
+            const int x = wave_total(sum[q]);
+            if (lane_id() == 0 && x)
+                atomicAdd(&all[q], x);
+            if (q < kNumTiers) {
+                const int y = wave_total(mine[q]);
+                if (lane_id() == 0 && y)
+                    atomicAdd(&before[q], y);
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < kNumTiers) {
+        int base = 0;
+        for (int q = 0; q < (int)threadIdx.x; q++)
+            base += all[q];
+        run[threadIdx.x] = base + before[threadIdx.x];
+        if (blockIdx.x == 0) {
+            p.ctl->list_begin[threadIdx.x] = base;
+            p.ctl->extra[threadIdx.x] = all[kNumTiers + threadIdx.x];
+            if (threadIdx.x == kNumTiers - 1)
+                p.ctl->list_begin[kNumTiers] = base + all[threadIdx.x];
+        }
+    }
     __syncthreads();
     const long long lo = (long long)blockIdx.x * p.per_block;
     const long long hi = min(lo + p.per_block, p.V);
     for (long long u0 = lo; u0 < hi; u0 += blockDim.x) {
         const long long u = u0 + threadIdx.x;
-        const int tier = u < hi ? plan_tier(p, u) : kTierNone;
-        int rank_in_wave[kNumTiers];
+        int parts = 1;
+        const int tier = u < hi ? plan_tier(p, u, parts) : kTierNone;
+        const bool split = __ballot(parts > 1) != 0;
+        int pos = 0;  // in the wave, within the tier
 #pragma unroll
         for (int t = 0; t < kNumTiers; t++) {
-            unsigned long long m = __ballot(tier == t);
-            rank_in_wave[t] = __builtin_amdgcn_mbcnt_hi((unsigned int)(m >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo((unsigned int)m, 0));
-            if (lane == 0)
-                wcount[t][wave] = __popcll(m);
+            int total, at;
+            if (split) {
+                const int x = tier == t ? parts : 0, incl = wave_scan_add(x);
+                total = readlane(incl, kWave - 1);
+                at = incl - x;
+            } else {
+                const unsigned long long m = __ballot(tier == t);
+                total = __popcll(m);
+                at = __builtin_amdgcn_mbcnt_hi((unsigned int)(m >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((unsigned int)m, 0));
+            }
+            if (lane_id() == 0)
+                wcount[t][wave] = total;
+            pos = tier == t ? at : pos;
         }
         __syncthreads();
         if (tier < kNumTiers) {
-            long long pos = run[tier] + rank_in_wave[tier];
+            pos += run[tier];
             for (int w = 0; w < wave; w++)
                 pos += wcount[tier][w];
-            p.list[pos] = (int32_t)u;
+            for (int q = 0; q < parts; q++)
+                p.list[pos + q] = (int32_t)u;
         }
         __syncthreads();
         if (threadIdx.x < kNumTiers) {
-            long long s = 0;
-            for (int w = 0; w < (int)(blockDim.x / kWave); w++)
-                s += wcount[threadIdx.x][w];
-            run[threadIdx.x] += s;
+            int sum = 0;
+            for (int w = 0; w < nwaves; w++)
+                sum += wcount[threadIdx.x][w];
+            run[threadIdx.x] += sum;
         }
         __syncthreads();
     }
@@ -1582,15 +1643,16 @@ __global__ void fill_u32_kernel(uint32_t *dst, uint32_t value, long long n)
 
 // ------------------------------------------------------------- wrappers
 template <typename OffT>
-hipError_t launch_plan(const PlanArgs<OffT> &p, int nblocks, hipStream_t stream)
+hipError_t launch_plan(PlanArgs<OffT> p, hipStream_t stream)
 {
-    if (nblocks > 0) {
-        hipLaunchKernelGGL(plan_count_kernel<OffT>, dim3(nblocks), dim3(256), 0, stream, p, nblocks);
-    }
-    hipLaunchKernelGGL(plan_scan_kernel<OffT>, dim3(1), dim3(1024), 0, stream, p, nblocks);
-    if (nblocks > 0) {
-        hipLaunchKernelGGL(plan_scatter_kernel<OffT>, dim3(nblocks), dim3(256), 0, stream, p, nblocks);
-    }
+    // small graphs: many small workgroups; large ones: at most kPlanBlocks
+    const int threads = p.V < (1 << 20) ? 256 : 1024;
+    const long long per = std::max<long long>(1, (p.V + (long long)threads * kPlanBlocks - 1) /
+                                                     ((long long)threads * kPlanBlocks));
+    p.per_block = (int)(per * threads);
+    const int nblocks = (int)std::max<long long>(1, (p.V + p.per_block - 1) / p.per_block);
+    hipLaunchKernelGGL(plan_count_kernel<OffT>, dim3(nblocks), dim3(threads), 0, stream, p);
+    hipLaunchKernelGGL(plan_scatter_kernel<OffT>, dim3(nblocks), dim3(threads), 0, stream, p, nblocks);
     return hipGetLastError();
 }
 
@@ -1681,8 +1743,8 @@ hipError_t launch_fill_u32(uint32_t *dst, uint32_t value, long long n, hipStream
     return hipGetLastError();
 }
 
-template hipError_t launch_plan<int32_t>(const PlanArgs<int32_t> &, int, hipStream_t);
-template hipError_t launch_plan<int64_t>(const PlanArgs<int64_t> &, int, hipStream_t);
+template hipError_t launch_plan<int32_t>(PlanArgs<int32_t>, hipStream_t);
+template hipError_t launch_plan<int64_t>(PlanArgs<int64_t>, hipStream_t);
 template hipError_t launch_count<int32_t>(const TcArgs<int32_t> &, int, int, size_t, int, bool,
                                           hipStream_t);
 template hipError_t launch_count<int64_t>(const TcArgs<int64_t> &, int, int, size_t, int, bool,

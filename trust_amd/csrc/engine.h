@@ -291,6 +291,14 @@ int core_enqueue(Ctx *ctx, TcCtl *ctl, hipStream_t s);
 void core_drop(Ctx *ctx);
 // core_drop and free the core's device memory (a synchronised stream)
 void core_release(Ctx *ctx);
+// A graph whose top out-degree is under 24 times the mean takes the
+// reference walk on every family measured (R-MAT 10-18, Chung-Lu, ER, BA:
+// 1.8 to 19 times; R-MAT 20 and up, which take the short side: 27 and up).
+// Only the order of the passes follows from it: reference_pass yields the
+// probe totals that decide, and with `starts` the reference walk's start
+// index (ctx->ref_built) unless there is no room for it.
+bool walk_probably_reference(const Ctx *ctx);
+int reference_pass(Ctx *ctx, bool starts);
 int walk_index_count(Ctx *ctx);
 int walk_index_build(Ctx *ctx);
 // Builds the walk of a tile from its device CSR and the global out-degrees
@@ -298,6 +306,8 @@ int walk_index_build(Ctx *ctx);
 template <typename OffT>
 int tile_walk_build(Ctx *ctx, const OffT *beg, const int32_t *adj, long long rows, long long cols,
                     const int32_t *degR, const int32_t *degC, TileWalk &tw);
+// Rows per wave of the passes over a CSR of `rows` rows (walk_index.hip).
+int rows_per_wave(long long rows, int num_cus);
 // Whether a tile walk with `cols` column vertices fits the binned build.
 int tile_walk_bins_ok(long long cols);
 

@@ -433,7 +433,7 @@ static int index_begin(Ctx *ctx, ResidentRun &R)
 // probe totals and the in-walk rows depend on the graph alone, so a context
 // makes them once per loaded graph (or again under TRUST_FLAG_FRESH_INDEX);
 // the count that makes them includes their device time in its seconds.
-static int prepare_side(Ctx *ctx, bool force, ResidentRun &R)
+static int prepare_side(Ctx *ctx, bool force, bool starts, ResidentRun &R)
 {
     DevCsr &g = ctx->g;
     // The binned build needs scratch beyond the index itself (per-edge d+,
@@ -467,10 +467,18 @@ static int prepare_side(Ctx *ctx, bool force, ResidentRun &R)
         return walk_index_count(ctx);
     };
     int rc;
+    bool made_starts = false;  // here, for the reference walk
     if (!force && !ctx->side_stats_ready) {
         if ((rc = index_begin(ctx, R)))
             return rc;
-        if (binned) {
+        const bool ref_first = walk_probably_reference(ctx);
+        if (ref_first) {
+            made_starts = !ctx->ref_built;
+            if ((rc = reference_pass(ctx, starts && made_starts)))
+                return rc;
+            made_starts = made_starts && ctx->ref_built;
+        }
+        if (binned && !ref_first) {
             // the binned build's count pass yields the probe totals too
             rc = count_pass();
             if (rc == TRUST_ERR_OOM)
@@ -478,7 +486,7 @@ static int prepare_side(Ctx *ctx, bool force, ResidentRun &R)
             if (rc)
                 return rc;
         }
-        if (!binned) {
+        if (!binned && !ref_first) {
             rc = ctx->side_stats.ensure(4 * sizeof(unsigned long long));
             if (rc)
                 return rc;
@@ -499,6 +507,11 @@ static int prepare_side(Ctx *ctx, bool force, ResidentRun &R)
     }
     R.side = force || (double)ctx->side_w_short <= kShortWalkShare * (double)ctx->side_w_ref;
     if (R.side && !ctx->side_built) {
+        if (made_starts) {  // the short side after all
+            HIPCHK(hipStreamSynchronize(ctx->stream));
+            ctx->ref_ent.release();
+            ctx->ref_built = false;
+        }
         if ((rc = index_begin(ctx, R)))
             return rc;
         const size_t ob = g.off64 ? sizeof(int64_t) : sizeof(int32_t);
@@ -610,7 +623,7 @@ int ensure_walk_index(Ctx *ctx)
     if (ctx->g.V <= 0 || ctx->g.E <= 0 || ctx->side_built)
         return TRUST_OK;
     ResidentRun R;
-    int rc = prepare_side(ctx, true, R);
+    int rc = prepare_side(ctx, true, false, R);
     if (!rc)
         HIPCHK(hipStreamSynchronize(ctx->stream));
     return rc;
@@ -665,7 +678,9 @@ int prepare_resident(Ctx *ctx, const trust_params &p, int mode, ResidentRun &R)
     R.index_ev = false;
     R.index_seconds = 0;
     if (!(p.flags & TRUST_FLAG_REFERENCE_WALK) && g.V > 0 && g.E > 0) {
-        rc = prepare_side(ctx, (p.flags & TRUST_FLAG_SHORT_WALK) != 0, R);
+        rc = prepare_side(ctx, (p.flags & TRUST_FLAG_SHORT_WALK) != 0,
+                          !(p.flags & TRUST_FLAG_OFFSET_LOOKUP) && !g.off64 &&
+                              ctx->batch_ngraphs == 0, R);
         if (rc)
             return rc;
         R.core = R.side && ctx->core.active;

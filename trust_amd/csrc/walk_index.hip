@@ -15,7 +15,7 @@
 // the hot path are LDS atomics, and every global store lands either in a
 // run that one workgroup owns or inside one bin's rows:
 //
-//   A   count    one pass over the CSR, 64 rows per wave in coalesced
+//   A   count    one pass over the CSR, up to 64 rows per wave in coalesced
 //                64-wide windows: both walks' probe totals (which decide the
 //                walk), each row's kept out-entries (per-wave LDS counters,
 //                one row per lane) and, per workgroup, an LDS histogram of
@@ -103,13 +103,14 @@ struct WiPassArgs {
     const OffT *beg;
     const int32_t *adj;
     long long V;  // rows
+    int rows;     // rows per wave and step, at most 64 (rows_per_wave)
     int nbins;
     // tiles: global out-degree of each row's vertex and of each column's
     // vertex (the resident graph takes both from beg)
     const int32_t *degR, *degC;
     int *kept;                    // A: out-entries per row
     int *M;                       // A: in-entries per bin and workgroup, bin-major
-    unsigned long long *stats;    // A: probes of both walks (resident graph)
+    unsigned long long *stats;    // A: per workgroup, probes of both walks and what the core takes
     // resident graph: d+ of each entry's vertex (edges of rows with d+ >= 2),
     // written by A, read by B in place of a second pair of offset lookups;
     // -1 marks an edge the dense core counts
@@ -128,7 +129,7 @@ struct WiPassArgs {
     typename WiFmt<OffT, kTile>::Rec *recs;
 };
 
-// Passes A (kPass 0) and B (kPass 1).  Grid-stride over 64-row groups by
+// Passes A (kPass 0) and B (kPass 1).  Grid-stride over groups of rows by
 // global wave id: both passes give every row to the same workgroup, which
 // is what lets pass B write at the offsets pass A's histograms produced.
 template <typename OffT, int kPass, bool kTile>
@@ -155,9 +156,9 @@ __global__ void __launch_bounds__(kPassThreads) wi_pass_kernel(WiPassArgs<OffT, 
         mark[k * kWave + lane] = 0;
     __syncthreads();
     unsigned long long w_ref = 0, w_short = 0, w_dense = 0, n_dense = 0;
-    const long long step = (long long)G * kPassWaves * kWave;
-    for (long long u0 = ((long long)blockIdx.x * kPassWaves + wave) * kWave; u0 < V; u0 += step) {
-        const int n = (int)min((long long)kWave, V - u0);
+    const long long step = (long long)G * kPassWaves * a.rows;
+    for (long long u0 = ((long long)blockIdx.x * kPassWaves + wave) * a.rows; u0 < V; u0 += step) {
+        const int n = (int)min((long long)a.rows, V - u0);
         // lane i < n holds row u0 + i; lane n (if any) the end of the range
         const OffT s = beg[u0 + min(lane, n)];
         const int d = lane < n ? (int)(beg[u0 + lane + 1] - s) : 0;
@@ -276,21 +277,100 @@ __global__ void __launch_bounds__(kPassThreads) wi_pass_kernel(WiPassArgs<OffT, 
         __syncthreads();
         for (int b = threadIdx.x; b < a.nbins; b += blockDim.x)
             a.M[(long long)b * G + blockIdx.x] = (int)bins[b];
+        // per workgroup, summed on the host: 8192 waves adding to the same
+        // four totals took 130 us of a pass over R-MAT 16
         if constexpr (!kTile) {
+            __shared__ unsigned long long sums[4];
+            if (threadIdx.x < 4)
+                sums[threadIdx.x] = 0;
+            __syncthreads();
             w_ref = wave_sum(w_ref);
             w_short = wave_sum(w_short);
             w_dense = wave_sum(w_dense);
             n_dense = wave_sum(n_dense);
-            if (lane == 0 && w_ref) {
-                atomicAdd(a.stats, w_ref);
-                atomicAdd(a.stats + 1, w_short);
-                if (n_dense) {
-                    atomicAdd(a.stats + 2, w_dense);
-                    atomicAdd(a.stats + 3, n_dense);
-                }
-            }
+            if (lane < 4)
+                atomicAdd(sums + lane, lane == 0 ? w_ref : lane == 1 ? w_short
+                                       : lane == 2 ? w_dense : n_dense);
+            __syncthreads();
+            if (threadIdx.x < 4)
+                a.stats[4 * blockIdx.x + threadIdx.x] = sums[threadIdx.x];
         }
     }
+}
+
+// Both walks' probe totals of a graph that will probably take the reference
+// walk, and (ent) that walk's start index, in one pass: pass A's histogram,
+// per-row counts and per-edge d+ are the short-side walk's.
+template <typename OffT>
+__global__ void __launch_bounds__(kPassThreads)
+ref_pass_kernel(const OffT *__restrict__ beg, const int32_t *__restrict__ adj, long long V, int rows,
+                WalkEntry<OffT> *__restrict__ ent, unsigned long long *__restrict__ stats)
+{
+    __shared__ int mark_s[kPassWaves][kWave * kWin];
+    __shared__ unsigned long long sums[2];
+    const int wave = threadIdx.x / kWave, lane = lane_id();
+    int *mark = mark_s[wave];
+    for (int k = 0; k < kWin; k++)
+        mark[k * kWave + lane] = 0;
+    if (threadIdx.x < 2)
+        sums[threadIdx.x] = 0;
+    __syncthreads();
+    unsigned long long w_ref = 0, w_short = 0;
+    const long long step = (long long)gridDim.x * kPassWaves * rows;
+    for (long long u0 = ((long long)blockIdx.x * kPassWaves + wave) * rows; u0 < V; u0 += step) {
+        const int n = (int)min((long long)rows, V - u0);
+        const OffT s = beg[u0 + min(lane, n)];
+        const int d = lane < n ? (int)(beg[u0 + lane + 1] - s) : 0;
+        const long long e0 = (long long)readlane(s, 0);
+        const long long e1 = n == kWave ? (long long)readlane(s, 63) + readlane(d, 63)
+                                        : (long long)readlane(s, n);
+        int carry = 0;
+        for (long long p = e0; p < e1; p += kWave * kWin) {
+            if (d > 0 && (long long)s >= p && (long long)s < p + kWave * kWin)
+                mark[(int)((long long)s - p)] = lane;
+            wave_sync();
+            int own[kWin], v[kWin];
+#pragma unroll
+            for (int k = 0; k < kWin; k++) {
+                own[k] = max(wave_scan_max(mark[k * kWave + lane]), carry);
+                carry = readlane(own[k], 63);
+                const long long pos = p + k * kWave + lane;
+                v[k] = pos < e1 ? adj[pos] : -1;
+            }
+            wave_sync();
+            OffT bv[kWin], ev[kWin];
+#pragma unroll
+            for (int k = 0; k < kWin; k++) {
+                mark[k * kWave + lane] = 0;
+                bv[k] = ev[k] = 0;
+                if (v[k] >= 0) {
+                    bv[k] = beg[v[k]];
+                    ev[k] = beg[v[k] + 1];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < kWin; k++) {
+                const int du = shfl_idx(d, own[k]);
+                if (v[k] < 0)
+                    continue;
+                const int dv = (int)(ev[k] - bv[k]);
+                if (ent)
+                    ent[p + k * kWave + lane] = WalkEntry<OffT>{bv[k], dv};
+                if (du >= 2) {
+                    w_ref += (unsigned long long)dv;
+                    w_short += (unsigned long long)min(du, dv);
+                }
+            }
+            wave_sync();
+        }
+    }
+    w_ref = wave_sum(w_ref);
+    w_short = wave_sum(w_short);
+    if (lane < 2)
+        atomicAdd(sums + lane, lane == 0 ? w_ref : w_short);
+    __syncthreads();
+    if (threadIdx.x < 2)
+        stats[4 * blockIdx.x + threadIdx.x] = sums[threadIdx.x];
 }
 
 // C1: ranks within one slice; in-counts of the bin's targets.
@@ -455,16 +535,17 @@ wi_place_kernel(const WiSlice *__restrict__ sl, const WiChunk *__restrict__ chun
 template <typename OffT>
 __global__ void __launch_bounds__(256)
 wi_outcopy_kernel(const OffT *__restrict__ outBeg, const OffT *__restrict__ begX, long long V,
-                  const WalkEntry<OffT> *__restrict__ tmpOut, WalkEntry<OffT> *__restrict__ entX)
+                  const WalkEntry<OffT> *__restrict__ tmpOut, WalkEntry<OffT> *__restrict__ entX,
+                  int rows)
 {
     __shared__ int mark_s[4][kWave];
     const int wave = threadIdx.x / kWave, lane = lane_id();
     int *mark = mark_s[wave];
     mark[lane] = 0;
-    const long long step = (long long)gridDim.x * (blockDim.x / kWave) * kWave;
-    for (long long u0 = ((long long)blockIdx.x * (blockDim.x / kWave) + wave) * kWave; u0 < V;
+    const long long step = (long long)gridDim.x * (blockDim.x / kWave) * rows;
+    for (long long u0 = ((long long)blockIdx.x * (blockDim.x / kWave) + wave) * rows; u0 < V;
          u0 += step) {
-        const int n = (int)min((long long)kWave, V - u0);
+        const int n = (int)min((long long)rows, V - u0);
         const OffT s = outBeg[u0 + min(lane, n)];
         const OffT e = lane < n ? outBeg[u0 + lane + 1] : s;
         const OffT bx = lane < n ? begX[u0 + lane] : (OffT)0;
@@ -627,15 +708,43 @@ int walk_bins(long long V) { return (int)((V + kBinSize - 1) / kBinSize); }
 
 bool walk_index_binned(const Ctx *ctx) { return ctx->g.V > 0 && walk_bins(ctx->g.V) <= kMaxBins; }
 
-// Pass A and the scans over a CSR of `rows` rows whose in-entries target
-// [0, cols): kept and outBeg (rows + 1) on the device; the bins' first
-// records, the out-entry total and (resident graph) both walks' probe
-// totals, then the probes and edges the dense core took, on the host.
-// Synchronises.
+// Rows that a wave takes at a time in the passes over the CSR: 64, fewer
+// where that leaves a wave with less than 16 groups of them.  The rows of
+// the top degree class stand together, 64 of them hold tens of thousands of
+// entries, and with few groups the waves that get them are the last ones
+// (64 at a time: pass A 150 us at R-MAT 16, 590 at R-MAT 20).
+int rows_per_wave(long long rows, int num_cus)
+{
+    const long long groups = 16ll * 32 * num_cus;  // 32 waves per CU
+    int n = 8;
+    while (n < kWave && groups * n < rows)
+        n *= 2;
+    return n;
+}
+
+// Sums of the passes' per-workgroup totals (synchronises).
+static int read_stats(Ctx *ctx, int groups, unsigned long long out[4])
+{
+    std::vector<unsigned long long> h(4 * (size_t)groups);
+    if (groups > 0)
+        HIPCHK(hipMemcpyAsync(h.data(), ctx->side_stats.p, sizeof(h[0]) * h.size(),
+                              hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    for (int k = 0; k < 4; k++)
+        out[k] = 0;
+    for (size_t i = 0; i < h.size(); i++)
+        out[i % 4] += h[i];
+    return TRUST_OK;
+}
+
+// Pass A over a CSR of `rows` rows whose in-entries target [0, cols): kept
+// and the histograms on the device; with stats_out (resident graph) both
+// walks' probe totals, then the probes and edges the dense core took, on the
+// host (synchronises).
 template <typename OffT, bool kTile>
 static int wi_count(Ctx *ctx, const OffT *beg, const int32_t *adj, long long rows, long long cols,
-                    const int32_t *degR, const int32_t *degC, int *kept, OffT *outBeg,
-                    unsigned long long stats_out[4], int32_t *dvE)
+                    const int32_t *degR, const int32_t *degC, int *kept,
+                    unsigned long long *stats_out, int32_t *dvE)
 {
     WalkIndexState &w = ctx->wi;
     const int nbins = std::max(1, walk_bins(cols));
@@ -655,15 +764,15 @@ static int wi_count(Ctx *ctx, const OffT *beg, const int32_t *adj, long long row
         (rc = w.bin_start.ensure(sizeof(long long) * (size_t)(nbins + 1))) ||
         (rc = w.bsum.ensure(sizeof(long long) *
                             (size_t)(scan_blocks(std::max(nM, std::max(rows, cols))) + 1))) ||
-        (rc = ctx->side_stats.ensure(4 * sizeof(unsigned long long))))
+        (rc = ctx->side_stats.ensure(4 * sizeof(unsigned long long) * (size_t)G)))
         return rc;
     unsigned long long *st = (unsigned long long *)ctx->side_stats.p;
-    HIPCHK(launch_fill_u32((uint32_t *)st, 0u, 8, ctx->stream));
     WiPassArgs<OffT, kTile> pa;
     memset(&pa, 0, sizeof(pa));
     pa.beg = beg;
     pa.adj = adj;
     pa.V = rows;
+    pa.rows = rows_per_wave(rows, ctx->num_cus);
     pa.nbins = nbins;
     pa.degR = degR;
     pa.degC = degC;
@@ -691,26 +800,79 @@ static int wi_count(Ctx *ctx, const OffT *beg, const int32_t *adj, long long row
     } else {
         HIPCHK(launch_fill_u32((uint32_t *)w.M.p, 0u, nM, ctx->stream));
     }
-    HIPCHK(launch_scan<int64_t>((const int *)w.M.p, nullptr, nM, (long long *)w.bsum.p,
-                                (int64_t *)w.O.p, ctx->stream));
+    w.grid = G;
+    w.nbins = nbins;
+    return stats_out ? read_stats(ctx, rows > 0 ? G : 0, stats_out) : TRUST_OK;
+}
+
+// Totals of a reference-walk graph (and its start index, unless ent is null).
+template <typename OffT>
+static int ref_pass(Ctx *ctx, WalkEntry<OffT> *ent, unsigned long long *stats_out)
+{
+    const DevCsr &g = ctx->g;
+    const int rows = rows_per_wave(g.V, ctx->num_cus);
+    const long long per = (long long)rows * kPassWaves;
+    const int G = (int)std::min<long long>((g.V + per - 1) / per, 2ll * ctx->num_cus);
+    if (int rc = ctx->side_stats.ensure(4 * sizeof(unsigned long long) * (size_t)G))
+        return rc;
+    hipLaunchKernelGGL(ref_pass_kernel<OffT>, dim3(G), dim3(kPassThreads), 0, ctx->stream,
+                       (const OffT *)g.beg.p, (const int32_t *)g.adj.p, (long long)g.V, rows, ent,
+                       (unsigned long long *)ctx->side_stats.p);
+    HIPCHK(hipGetLastError());
+    return read_stats(ctx, G, stats_out);
+}
+
+bool walk_probably_reference(const Ctx *ctx)
+{
+    const DevCsr &g = ctx->g;
+    return (double)g.max_deg * (double)g.V < 24.0 * (double)g.E;
+}
+
+int reference_pass(Ctx *ctx, bool starts)
+{
+    const DevCsr &g = ctx->g;
+    unsigned long long h[4];
+    int rc;
+    if (g.off64) {
+        rc = ref_pass<int64_t>(ctx, nullptr, h);
+    } else {
+        // without room for the index the totals come alone
+        if (starts && ctx->ref_ent.ensure(sizeof(WalkEntry<int32_t>) * (size_t)g.E))
+            starts = false;
+        rc = ref_pass<int32_t>(ctx, starts ? (WalkEntry<int32_t> *)ctx->ref_ent.p : nullptr, h);
+    }
+    if (rc)
+        return rc;
+    ctx->side_w_ref = h[0];
+    ctx->side_w_short = h[1];
+    ctx->side_stats_ready = true;
+    ctx->ref_built = ctx->ref_built || (starts && !g.off64);
+    return TRUST_OK;
+}
+
+// The scans after pass A: kept -> outBeg (rows + 1), the histograms -> each
+// workgroup's first record in each bin, all on the device; the bins' first
+// records and the out-entry total on the host.  Synchronises.  Apart from
+// pass A because a count that takes the reference walk needs only its totals:
+// seven launches and two copies less (50 us) on small graphs.
+template <typename OffT>
+static int wi_offsets(Ctx *ctx, long long rows, const int *kept, OffT *outBeg)
+{
+    WalkIndexState &w = ctx->wi;
+    const int G = w.grid, nbins = w.nbins;
+    HIPCHK(launch_scan<int64_t>((const int *)w.M.p, nullptr, (long long)nbins * G,
+                                (long long *)w.bsum.p, (int64_t *)w.O.p, ctx->stream));
     hipLaunchKernelGGL(wi_bin_starts_kernel, dim3((unsigned)((nbins + 256) / 256)), dim3(256), 0,
                        ctx->stream, (const long long *)w.O.p, G, nbins, (long long *)w.bin_start.p);
     HIPCHK(hipGetLastError());
     HIPCHK(launch_scan<OffT>(kept, nullptr, rows, (long long *)w.bsum.p, outBeg, ctx->stream));
     w.bin_start_h.resize((size_t)nbins + 1);
-    unsigned long long h[4];
     OffT out_total = 0;
-    HIPCHK(hipMemcpyAsync(h, st, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipMemcpyAsync(w.bin_start_h.data(), w.bin_start.p, sizeof(long long) * (nbins + 1),
                           hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipMemcpyAsync(&out_total, outBeg + rows, sizeof(OffT), hipMemcpyDeviceToHost,
                           ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (stats_out)
-        for (int k = 0; k < 4; k++)
-            stats_out[k] = h[k];
-    w.grid = G;
-    w.nbins = nbins;
     w.out_total = (int64_t)out_total;
     return TRUST_OK;
 }
@@ -811,6 +973,7 @@ static int wi_build(Ctx *ctx, const OffT *beg, const int32_t *adj, long long row
     pa.beg = beg;
     pa.adj = adj;
     pa.V = rows;
+    pa.rows = rows_per_wave(rows, ctx->num_cus);
     pa.nbins = nbins;
     pa.degR = degR;
     pa.degC = degC;
@@ -844,10 +1007,11 @@ static int wi_build(Ctx *ctx, const OffT *beg, const int32_t *adj, long long row
     }
     if constexpr (!kTile) {
         if (x_out > 0) {
-            const int blocks = (int)std::min<long long>((rows + 4 * kWave - 1) / (4 * kWave), 16384ll);
+            const int per = rows_per_wave(rows, ctx->num_cus);
+            const int blocks = (int)std::min<long long>((rows + 4 * per - 1) / (4 * per), 16384ll);
             hipLaunchKernelGGL(wi_outcopy_kernel<OffT>, dim3(blocks), dim3(256), 0, ctx->stream,
                                outBeg, (const OffT *)begX, rows, (const WalkEntry<OffT> *)tmpOut,
-                               entX);
+                               entX, per);
             HIPCHK(hipGetLastError());
         }
     }
@@ -861,14 +1025,12 @@ static int count_pass_t(Ctx *ctx)
     WalkIndexState &w = ctx->wi;
     const long long V = g.V;
     int rc;
-    if ((rc = w.out_beg.ensure(sizeof(OffT) * (size_t)(V + 1))) ||
-        (rc = w.dv.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(g.E, 1))) ||
+    if ((rc = w.dv.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(g.E, 1))) ||
         (rc = ctx->side_cnt.ensure(2 * sizeof(int) * (size_t)V)))
         return rc;
     unsigned long long h[4];
     rc = wi_count<OffT, false>(ctx, (const OffT *)g.beg.p, (const int32_t *)g.adj.p, V, V, nullptr,
-                               nullptr, (int *)ctx->side_cnt.p + V, (OffT *)w.out_beg.p, h,
-                               (int32_t *)w.dv.p);
+                               nullptr, (int *)ctx->side_cnt.p + V, h, (int32_t *)w.dv.p);
     if (rc)
         return rc;
     ctx->side_w_ref = h[0];
@@ -891,9 +1053,12 @@ static int build_t(Ctx *ctx)
     DevCsr &g = ctx->g;
     WalkIndexState &w = ctx->wi;
     const long long V = g.V;
-    const long long x_in = w.bin_start_h[(size_t)w.nbins], x_out = w.out_total;
     const size_t ob = sizeof(OffT);
     int rc;
+    if ((rc = w.out_beg.ensure(ob * (size_t)(V + 1))) ||
+        (rc = wi_offsets<OffT>(ctx, V, (const int *)ctx->side_cnt.p + V, (OffT *)w.out_beg.p)))
+        return rc;
+    const long long x_in = w.bin_start_h[(size_t)w.nbins], x_out = w.out_total;
     if ((rc = w.tmp_out.ensure(2 * ob * (size_t)std::max<long long>(x_out, 1))) ||
         (rc = ctx->side_beg.ensure(ob * (size_t)(V + 1))) ||
         (rc = ctx->side_ent.ensure(2 * ob * (size_t)std::max<long long>(x_in + x_out, 1))))
@@ -933,9 +1098,8 @@ int tile_walk_build(Ctx *ctx, const OffT *beg, const int32_t *adj, long long row
         (rc = ctx->side_cnt.ensure(sizeof(int) * (size_t)(rows + cols))))
         return rc;
     int *kept = (int *)ctx->side_cnt.p, *incnt = kept + rows;
-    rc = wi_count<OffT, true>(ctx, beg, adj, rows, cols, degR, degC, kept, (OffT *)tw.out_beg.p,
-                              nullptr, nullptr);
-    if (rc)
+    if ((rc = wi_count<OffT, true>(ctx, beg, adj, rows, cols, degR, degC, kept, nullptr, nullptr)) ||
+        (rc = wi_offsets<OffT>(ctx, rows, kept, (OffT *)tw.out_beg.p)))
         return rc;
     WalkIndexState &w = ctx->wi;
     tw.x_out = w.out_total;

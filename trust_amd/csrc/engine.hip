@@ -280,8 +280,9 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
         return rc;
     // a list made elsewhere, and the instrumented mode's per-vertex outputs,
     // know whole vertices only
-    const int part_entries =
-        preplanned || seg || (mode & ~kProbeDeep) == kModeInstr ? 0 : walk_part_entries(views.entries);
+    const bool whole = preplanned || seg || (mode & ~kProbeDeep) == kModeInstr;
+    const int part_entries = whole ? 0 : walk_part_entries(views.entries);
+    const int wave_part = whole ? 0 : walk_wave_part(views.entries, V);
     if (L.spill_groups > 0) {
         rc = ctx->spill.ensure(sizeof(int32_t) * (size_t)L.spill_slots * L.spill_groups);
         if (rc)
@@ -302,6 +303,7 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
         pa.force_spill = (p.flags & TRUST_FLAG_FORCE_SPILL) ? 1 : 0;
         pa.wave_only = (p.flags & TRUST_FLAG_WAVE_ONLY) ? 1 : 0;
         pa.part_entries = part_entries;
+        pa.wave_part = wave_part;
         pa.list = seg ? (int32_t *)seg->list : (int32_t *)ctx->list.p;
         pa.block_counts = (int *)ctx->block_counts.p;
         pa.ctl = ctl_dev;
@@ -347,6 +349,7 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
     }
     fill_args(a, ctx, views, p, L, L.main, ctl_dev, instr_cycles, instr_probes, seg);
     a.part_entries = part_entries;
+    a.wave_part = wave_part;
     a.spill_tier = -1;
     a.group_tier = kTierHub;
     a.wave_tier = kTierWave;
@@ -844,7 +847,7 @@ int finish_resident(Ctx *ctx, ResidentRun &R, const TcCtl &h, double t_plan, dou
                           : alg_bytes(g.V, g.E, h.probes, g.off64 && !R.segmented);
     r->n_spill = h.list_begin[kTierSpill + 1] - h.list_begin[kTierSpill];
     r->n_hub = group_vertices(h);  // big + hub
-    r->n_wave = h.list_begin[kTierWave + 1] - h.list_begin[kTierWave];
+    r->n_wave = wave_vertices(h);
     r->threads = L.main.threads;
     r->blocks = L.main.blocks;
     r->hub_slots = 1 << L.main.group_lg;

@@ -204,6 +204,7 @@ extern "C" int trust_count_csr_noalloc(const int64_t *beg_dev, const int32_t *ad
     pa.list = list;
     pa.block_counts = block_counts;
     pa.part_entries = walk_part_entries(E);
+    pa.wave_part = walk_wave_part(E, V);
     pa.ctl = ctl;
     HIPCHK(launch_plan<int32_t>(pa, s));
     TcArgs<int32_t> a;
@@ -213,6 +214,7 @@ extern "C" int trust_count_csr_noalloc(const int64_t *beg_dev, const int32_t *ad
     a.adjH = a.adjW = a.adjP = adj_dev;
     a.list = list;
     a.part_entries = walk_part_entries(E);
+    a.wave_part = walk_wave_part(E, V);
     a.spill_tier = -1;
     a.chunk_group = L.chunk_group;
     a.chunk_wave = L.chunk_wave;
@@ -262,7 +264,7 @@ extern "C" int trust_count_csr_noalloc(const int64_t *beg_dev, const int32_t *ad
         r->alg_bytes = alg_bytes(V, E, h.probes, false);
         r->n_spill = 0;
         r->n_hub = group_vertices(h);
-        r->n_wave = h.list_begin[kTierWave + 1] - h.list_begin[kTierWave];
+        r->n_wave = wave_vertices(h);
         r->threads = L.main.threads;
         r->blocks = L.main.blocks;
         r->hub_slots = 1 << L.main.group_lg;

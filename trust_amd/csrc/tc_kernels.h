@@ -72,6 +72,11 @@ struct alignas(128) TcCtl {
 };
 // Bytes of a control block that hold results (list bounds, sums).
 constexpr size_t kCtlHead = offsetof(TcCtl, wave_next);
+// Vertices of the wave tier.
+inline long long wave_vertices(const TcCtl &h)
+{
+    return h.list_begin[kTierWave + 1] - h.list_begin[kTierWave] - h.extra[kTierWave];
+}
 // Vertices of the workgroup tiers with LDS tables (big and hub).
 inline long long group_vertices(const TcCtl &h)
 {
@@ -121,6 +126,7 @@ struct TcArgs {
     int chunk_group;         // vertices per grab, spill/group tiers
     int chunk_wave;          // vertices per grab, wave tier (0: chosen by the kernel)
     int part_entries;        // walk entries of a workgroup-tier part (0: vertices are whole)
+    int wave_part;           // walk entries of a wave-tier part (0: vertices are whole)
     int pack_rows;           // rows a pack of the wave tier may hold (0, 1: no packs)
     int tag_shift;           // bits of an id (a pack's keys are id | row << tag_shift)
     int rank;
@@ -159,6 +165,7 @@ struct PlanArgs {
     int force_spill;
     int wave_only;
     int part_entries;   // see group_parts (0: vertices stay whole)
+    int wave_part;      // see wave_parts
     int32_t *list;      // V + kMaxExtra positions
     int *block_counts;  // kPlanBlocks x 2 kNumTiers
     int per_block;      // set by launch_plan
@@ -230,16 +237,16 @@ constexpr double kShortWalkShare = 0.45;
 // launch, whose workgroups are four times as large) fills one list position
 // per part, and each part builds the vertex's table for itself.
 // part_entries is 1/16384 of the walk, so that no part outlasts the count's
-// average workgroup and the list holds at most kMaxExtra more positions; at
+// average workgroup and the list holds at most kGroupExtra more positions; at
 // least 128, below which building the table costs more than the part's walk.
 constexpr int kBigPartLg = 2;
-constexpr long long kMaxExtra = 16384;
+constexpr long long kGroupExtra = 16384;
 inline int walk_part_entries(long long walk_entries)
 {
     if (walk_entries <= 0)
         return 0;
     int lg = 7;
-    while (lg < 28 && (kMaxExtra << lg) < walk_entries)
+    while (lg < 28 && (kGroupExtra << lg) < walk_entries)
         lg++;
     return 1 << lg;
 }
@@ -250,6 +257,31 @@ __host__ __device__ inline int group_parts(int dW, int part_entries, int tier)
     const int e = part_entries << (tier == kTierBig ? kBigPartLg : 0);
     return dW > e ? (dW + e - 1) / e : 1;
 }
+
+// Parts of the wave tier.  In a graph of less than 2 M walk entries the waves
+// that take a vertex of some 50 to 100 neighbours are the last to end, by
+// 150 us at R-MAT 16.  There a vertex fills a list position per `each` walk
+// entries, about a 32768th of the walk (a quarter of a wave's share) and 16
+// at least.  The position holds the part's number above kPartShift bits of
+// the vertex, so a vertex has at most kMaxWaveParts.
+constexpr int kPartShift = 26;
+constexpr int kMaxWaveParts = 32;
+constexpr long long kWaveExtra = 32768;
+inline int walk_wave_part(long long walk_entries, long long V)
+{
+    if (walk_entries <= 0 || walk_entries >= (2 << 20) || V > (1 << kPartShift))
+        return 0;
+    const long long e = (walk_entries + kWaveExtra - 1) / kWaveExtra;
+    return e < 16 ? 16 : (int)e;
+}
+__host__ __device__ inline int wave_parts(int dW, int each)
+{
+    if (each <= 0 || dW <= each)
+        return 1;
+    const int n = (dW + each - 1) / each;
+    return n < kMaxWaveParts ? n : kMaxWaveParts;
+}
+constexpr long long kMaxExtra = kGroupExtra + kWaveExtra;  // list positions beyond one per vertex
 
 // Packs of the wave tier (tc_kernels.hip): ids below `ids` leave the upper
 // bits of a 32-bit key for the row's number; the largest number is left out,

@@ -694,8 +694,9 @@ __device__ __forceinline__ void group_vertex(int u, int tier, long long at, int 
 
 // One wavefront counts vertex u with its own LDS table slice.
 template <typename OffT, int kMode, int kU>
-__device__ __forceinline__ void wave_vertex(ArgP<OffT> a, int u, OffT sH, int dH, OffT sW, int dW,
-                                            int *tab, int *mark, unsigned long long *sum)
+__device__ __forceinline__ void wave_vertex(ArgP<OffT> a, int u, bool first, OffT sH, int dH,
+                                            OffT sW, int dW, int *tab, int *mark,
+                                            unsigned long long *sum)
 {
     constexpr bool kInstr = kMode == kModeInstr;
     constexpr bool kTable = kMode != kModeGather;
@@ -728,7 +729,7 @@ __device__ __forceinline__ void wave_vertex(ArgP<OffT> a, int u, OffT sH, int dH
         wave_sync();
         linear = __ballot(failed) != 0;
         if (linear) {  // rebuild this vertex's table with linear probing
-            if (lane == 0 && a->force_linear != 1)
+            if (lane == 0 && a->force_linear != 1 && first)
                 atomicAdd(&a->ctl->rebuilds, 1ull);
             for (int i = lane; i < size; i += kWave)
                 tab[i] = kEmpty;
@@ -918,10 +919,15 @@ __device__ __forceinline__ int wave_next(ArgP<OffT> a, long long i, long long la
     constexpr bool kTable = kMode != kModeGather;
     const int lane = lane_id();
     const bool in = i + lane < last;
-    const int u = in ? a->list[i + lane] : 0;
+    int u = in ? a->list[i + lane] : 0;
     OffT sH = 0, sW = 0;
-    int dH = 0, dW = 0;
-    const bool same = a->begH == a->begW && a->adjH == a->adjW;
+    int dH = 0, dW = 0, part = 0;
+    const bool split = a->wave_part != 0;
+    const bool same = !split && a->begH == a->begW && a->adjH == a->adjW;
+    if (split) {
+        part = (int)((unsigned int)u >> kPartShift);
+        u &= (1 << kPartShift) - 1;
+    }
     if (in) {
         sH = a->begH[u];
         dH = (int)(a->begH[u + 1] - sH);
@@ -931,6 +937,12 @@ __device__ __forceinline__ int wave_next(ArgP<OffT> a, long long i, long long la
         } else {
             sW = a->begW[u];
             dW = (int)(a->endW[u] - sW);
+        }
+        if (split) {  // this part's share of the walk
+            const int parts = wave_parts(dW, a->wave_part);
+            const int each = (dW + parts - 1) / parts;
+            sW += (OffT)(part * each);
+            dW = max(0, min(each, dW - part * each));
         }
     }
     const int u0 = readlane(u, 0);
@@ -987,8 +999,8 @@ __device__ __forceinline__ int wave_next(ArgP<OffT> a, long long i, long long la
             }
         }
     }
-    wave_vertex<OffT, kMode, kU>(a, u0, readlane(sH, 0), readlane(dH, 0), readlane(sW, 0),
-                                 readlane(dW, 0), tab, mark, sum);
+    wave_vertex<OffT, kMode, kU>(a, u0, readlane(part, 0) == 0, readlane(sH, 0), readlane(dH, 0),
+                                 readlane(sW, 0), readlane(dW, 0), tab, mark, sum);
     return 1;
 }
 
@@ -1142,7 +1154,7 @@ tc_count_kernel(TcArgs<OffT>)
         // (larger chunks of a skewed list leave long ones for the end)
         int chunk = a->chunk_wave;
         if (chunk <= 0)
-            chunk = max(1, min(kWave, (int)(items / (2ll * gridDim.x * nwaves))));
+            chunk = a->wave_part ? 1 : max(1, min(kWave, (int)(items / (2ll * gridDim.x * nwaves))));
         const unsigned int n = rank_chunks(items, chunk, a->rank, a->nranks);
         constexpr bool kBatch = kMode == kModeBatch;
         constexpr int kShards = kBatch ? kXcds : kWaveShards;
@@ -1197,6 +1209,8 @@ __device__ __forceinline__ int plan_tier(const PlanArgs<OffT> &p, long long u, i
         parts = group_parts((int)dW, p.part_entries, kTierHub);
         return kTierHub;
     }
+    if (p.wave_part)
+        parts = wave_parts((int)dW, p.wave_part);
     return kTierWave;
 }
 
@@ -1321,7 +1335,7 @@ __global__ void __launch_bounds__(1024) plan_scatter_kernel(PlanArgs<OffT> p, in
             for (int w = 0; w < wave; w++)
                 pos += wcount[tier][w];
             for (int q = 0; q < parts; q++)
-                p.list[pos + q] = (int32_t)u;
+                p.list[pos + q] = tier == kTierWave ? (int32_t)u | q << kPartShift : (int32_t)u;
         }
         __syncthreads();
         if (threadIdx.x < kNumTiers) {

@@ -101,10 +101,12 @@ typedef struct trust_params {
      * core, and the walk leaves them out.  The core is the core_vertices
      * highest estimated degrees, closed under out-neighbours while it stays
      * within 32768 vertices.  A per-graph index like the walk rows, made by
-     * the first count that uses it.  core_vertices: 0 automatic (16384 for
-     * single graphs of at least 2^23 edges counted by one logical rank, else
-     * none), -1 none, else a power of two in [256, 16384].
-     * core_min_degree: 0 automatic (384), else >= 2. */
+     * the first count that uses it.  core_vertices: 0 automatic (for single
+     * graphs of at least 2^23 edges counted by one logical rank a power of two
+     * near twice the square root of the vertices, at most 16384; else none),
+     * -1 none, else a power of two in [256, 16384].
+     * core_min_degree: 0 automatic (a 48th of the core's vertices, 64 to 384),
+     * else >= 2. */
     int32_t reserved[3];   /* reserved[0]: a tile stream's device tile-cache slots (0: 2n+2) */
     int32_t core_vertices;
     int32_t core_min_degree;

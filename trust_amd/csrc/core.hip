@@ -61,19 +61,30 @@ constexpr int kCoreSeedMax = 16384;  // K0
 constexpr int kCoreSeedMin = 256;
 constexpr int kCoreMax = 32768;      // |C| (int16 ids; at most 32 slices of 32 words)
 constexpr int kCoreMaxSlices = 32;
-constexpr int kCoreGrabLg = 16;      // the lists kernel's grabs: 2^16 entries of adj
 constexpr int kCoreSteps = 6;        // closure steps
-// default t: R-MAT 26 fresh counts measured 253.6 ms at 256, 236.3 at 384,
-// 236.8 at 512; R-MAT 24 47.1, 47.5, 51.8 ms
-constexpr int kCoreMinDegree = 384;
+// The bound t on the degrees of dense edges, unless the caller gives one: a
+// dense edge costs nC / 8 bytes of bit rows whatever its probes, so t grows
+// with the core.  nC / 48 within [64, 384]: R-MAT 26 (17.9k vertices) fresh
+// counts measured 253.6 ms at t = 256, 236.3 at 384, 236.8 at 512; R-MAT 24
+// (12.9k) 44.4 ms at 192, 44.9 at 256, 45.3 at 384; counts of R-MAT 20 (6.2k)
+// 1.81 ms at 96, 1.38 at 128, 1.46 at 192, 2.09 at 384.
+constexpr int kCoreMinDegreeLow = 64, kCoreMinDegreeHigh = 384, kCorePerDegree = 48;
 constexpr int kCoreSample = 128;     // in-degree sampled every 128th entry
 constexpr int kCoreBins = 2048;      // histogram: est < 64 exact, then 64 bins per octave
 constexpr int kCorePart = 2048;      // dense targets per work item (longer lists are cut)
 constexpr int kCoreThreads = 256;
 constexpr int kCoreQueueStride = 32; // one 128-byte line per slice queue
-// misc words: [0] items of long lists (front of recs), [1] items of short
-// lists (back of recs), [2] closure additions, [3] bsrc slots taken, [4] rows
-// with d+ >= t, [5] the lists kernel's grab queue, then the slice queues
+// misc words: the slice queues follow at 64
+enum CoreMisc {
+    kCmLong = 0,     // items of long lists (front of recs)
+    kCmMembers = 2,  // vertices listed so far (past kCoreMax: the closure does not fit)
+    kCmSources = 3,  // candidate rows: bsrc slots, and an item each (back of recs)
+    kCmOver = 4,     // rows with d+ >= t
+    kCmTake = 8,     // the seed's size
+    kCmCut = 9,      // the seed's lowest histogram bin
+    kCmDegree = 10,  // t
+    kCmLevel = 16    // [k]: members before closure step k
+};
 constexpr int kCoreMiscWords = 64 + kCoreMaxSlices * kCoreQueueStride;
 
 // A work item: dense targets pool[lo + t0, lo + t1) of the source whose
@@ -136,64 +147,118 @@ core_hist_kernel(const OffT *__restrict__ beg, long long V, const int *__restric
             atomicAdd(&hist[b], h[b]);
 }
 
-// Membership states in flag[x]: 0 outside, 1 member whose out-list has been
-// added, 2 member to expand, 3 added by the running step.
+// The seed: the top bins, at most k0 vertices, no bin below bmin.  One
+// workgroup; cut = the lowest bin, take = its vertices.
+__global__ void __launch_bounds__(kCoreThreads)
+core_cut_kernel(const unsigned *__restrict__ hist, int bmin, unsigned k0, unsigned *__restrict__ misc)
+{
+    constexpr int kPer = kCoreBins / kCoreThreads;
+    __shared__ unsigned long long part[kCoreThreads];
+    __shared__ unsigned best, cut;
+    unsigned long long mine = 0;
+    for (int k = 0; k < kPer; k++)
+        mine += hist[threadIdx.x * kPer + k];
+    part[threadIdx.x] = mine;
+    if (threadIdx.x == 0) {
+        best = 0;
+        cut = kCoreBins;
+    }
+    __syncthreads();
+    // suffix sums of the threads' counts: above = the bins past this thread's
+    for (int off = 1; off < kCoreThreads; off <<= 1) {
+        const unsigned long long y = threadIdx.x + off < kCoreThreads ? part[threadIdx.x + off] : 0;
+        __syncthreads();
+        part[threadIdx.x] += y;
+        __syncthreads();
+    }
+    unsigned long long above = part[threadIdx.x] - mine;
+    for (int k = kPer - 1; k >= 0; k--) {
+        const int b = threadIdx.x * kPer + k;
+        above += hist[b];
+        if (above <= k0 && b >= bmin) {
+            atomicMin(&cut, (unsigned)b);
+            atomicMax(&best, (unsigned)above);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        misc[kCmTake] = best;
+        misc[kCmCut] = cut;
+        misc[kCmMembers] = 0;
+        misc[kCmLevel] = 0;
+    }
+}
+
+// Appends x to the member list for the lanes with `add`.
+__device__ __forceinline__ void core_append(bool add, int x, int *list, unsigned *members)
+{
+    const unsigned long long m = __ballot(add);
+    if (!m)
+        return;
+    unsigned at = 0;
+    if (lane_id() == 0)
+        at = atomicAdd(members, (unsigned)__popcll(m));
+    at = __builtin_amdgcn_readfirstlane(at) +
+         __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+    if (add && at < (unsigned)kCoreMax)
+        list[at] = x;
+}
+
+// flag[x] = 1 for the seed's vertices, 0 outside, and their list.
 template <typename OffT>
 __global__ void __launch_bounds__(kCoreThreads)
 core_seed_kernel(const OffT *__restrict__ beg, long long V, const int *__restrict__ din,
-                 int *__restrict__ flag, int bstar)
+                 int *__restrict__ flag, int *__restrict__ list, unsigned *__restrict__ misc)
 {
-    for (long long x = (long long)blockIdx.x * blockDim.x + threadIdx.x; x < V;
-         x += (long long)gridDim.x * blockDim.x)
-        flag[x] = core_bin(core_est(beg, din, x)) >= bstar ? 2 : 0;
+    const int cut = (int)misc[kCmCut];
+    const long long step = (long long)gridDim.x * blockDim.x;
+    for (long long x0 = (long long)blockIdx.x * blockDim.x + (threadIdx.x & ~(kWave - 1)); x0 < V;
+         x0 += step) {
+        const long long x = x0 + lane_id();
+        const bool in = x < V && core_bin(core_est(beg, din, x)) >= cut;
+        if (x < V)
+            flag[x] = in ? 1 : 0;
+        core_append(in, (int)x, list, misc + kCmMembers);
+    }
 }
 
-// One closure step: a wave takes 64 vertices and expands each member in
-// state 2 with the whole wave (its out-neighbours outside join in state 3).
+// Members listed before step k (the list's end as the step begins).
+__global__ void core_level_kernel(unsigned *__restrict__ misc, int k)
+{
+    misc[kCmLevel + k + 1] = min(misc[kCmMembers], (unsigned)kCoreMax + 1u);
+}
+
+// Closure step k: a wave per member that step k - 1 added; its
+// out-neighbours outside join the list.  Nothing once the list is full.
 template <typename OffT>
 __global__ void __launch_bounds__(kCoreThreads)
-core_expand_kernel(const OffT *__restrict__ beg, const int32_t *__restrict__ adj, long long V,
-                   int *__restrict__ flag, unsigned *__restrict__ added)
+core_expand_kernel(const OffT *__restrict__ beg, const int32_t *__restrict__ adj,
+                   int *__restrict__ flag, int *__restrict__ list, unsigned *__restrict__ misc, int k)
 {
     constexpr int kWaves = kCoreThreads / kWave;
-    const int wave = threadIdx.x / kWave, lane = lane_id();
-    const long long step = (long long)gridDim.x * kWaves * kWave;
-    unsigned n_add = 0;
-    for (long long x0 = ((long long)blockIdx.x * kWaves + wave) * kWave; x0 < V; x0 += step) {
-        const long long x = x0 + lane;
-        const int f = x < V ? flag[x] : 0;
-        unsigned long long todo = __ballot(f == 2);
-        if (f == 2)
-            flag[x] = 1;
-        while (todo) {
-            const int i = __builtin_ctzll(todo);
-            todo &= todo - 1;
-            const long long lo = (long long)beg[x0 + i], hi = (long long)beg[x0 + i + 1];
-            for (long long p = lo + lane; p < hi; p += kWave) {
-                const int w = adj[p];
-                if (flag[w] == 0 && atomicCAS(&flag[w], 0, 3) == 0)
-                    n_add++;
-            }
+    const unsigned lo = misc[kCmLevel + k], hi = misc[kCmLevel + k + 1];
+    if (hi > (unsigned)kCoreMax)
+        return;
+    const int lane = lane_id();
+    for (unsigned m = lo + blockIdx.x * kWaves + threadIdx.x / kWave; m < hi;
+         m += gridDim.x * kWaves) {
+        const int x = __builtin_amdgcn_readfirstlane(list[m]);
+        const long long p0 = (long long)beg[x], p1 = (long long)beg[x + 1];
+        for (long long p = p0; p < p1; p += kWave) {
+            const int w = p + lane < p1 ? adj[p + lane] : -1;
+            const bool add = w >= 0 && flag[w] == 0 && atomicCAS(&flag[w], 0, 1) == 0;
+            core_append(add, w, list, misc + kCmMembers);
         }
     }
-    n_add = (unsigned)wave_sum((unsigned long long)n_add);
-    if (lane == 0 && n_add)
-        atomicAdd(added, n_add);
 }
 
-// After a step: state 3 -> 2 (the next step expands them).  last: every
-// member -> 1 and everything else -> 0 (the scan's input).
-__global__ void __launch_bounds__(kCoreThreads)
-core_promote_kernel(long long V, int *__restrict__ flag, int last)
+// t of the core found, unless the caller gave one.
+__global__ void core_degree_kernel(unsigned *__restrict__ misc, int thr)
 {
-    for (long long x = (long long)blockIdx.x * blockDim.x + threadIdx.x; x < V;
-         x += (long long)gridDim.x * blockDim.x) {
-        const int f = flag[x];
-        if (last)
-            flag[x] = f != 0 ? 1 : 0;
-        else if (f == 3)
-            flag[x] = 2;
-    }
+    const int n = (int)min(misc[kCmMembers], (unsigned)kCoreMax);
+    misc[kCmDegree] = (unsigned)(thr > 0 ? thr
+                                         : min(max(n / kCorePerDegree, kCoreMinDegreeLow),
+                                               kCoreMinDegreeHigh));
 }
 
 // flag (0/1) and its exclusive scan -> cid (int16, -1 outside) and coreV
@@ -265,9 +330,14 @@ core_rows_kernel(const OffT *__restrict__ beg, const int32_t *__restrict__ adj,
 // turn: its core ids into an LDS bitmap, which checks for repeats and is the
 // row B(u) (stored to bsrc for a dense source), and its dense targets' ids
 // from the row's start of pool (pool has adj's indexing); then the row's
-// work items (targets cut into kCorePart pieces; rows with more than
-// kCorePart targets fill recs from the front, the others from the back, so
-// the long ones are handed out first).
+// work items, targets cut into kCorePart pieces.  A candidate row's slot b in
+// bsrc is also its place from the back of recs (an empty item where it is no
+// dense source, or has more than kCorePart targets: those fill recs from the
+// front, so that the long ones are handed out first).  With an atomic per
+// item the kernel ended no earlier than one counter took them: 11.5 ns each.
+//
+// R-MAT's long rows crowd at low ids, so a wave's share of the rows is those
+// that start in equal ranges of entries (grab_row), several ranges per wave.
 template <typename OffT>
 __global__ void __launch_bounds__(kCoreThreads)
 core_lists_kernel(const OffT *__restrict__ beg, const int32_t *__restrict__ adj, long long V,
@@ -288,28 +358,41 @@ core_lists_kernel(const OffT *__restrict__ beg, const int32_t *__restrict__ adj,
     for (int i = lane; i < words; i += kWave)
         seen[i] = 0;
     __syncthreads();
-    // R-MAT's long rows crowd at low ids: the grabs are equal ranges of
-    // entries (the rows starting in 2^16 entries of adj), from a queue
-    for (;;) {
-        unsigned q = 0;
-        if (lane == 0)
-            q = atomicAdd(&misc[5], 1u);
-        q = __builtin_amdgcn_readfirstlane(q);
-        if ((long long)q >= ngrab)
-            break;
+    // the workgroup's candidate rows, one atomic for their bsrc slots
+    __shared__ unsigned cand_s[kWaves], base_s;
+    unsigned ncand = 0;
+    const long long q0 = (long long)wave * gridDim.x + blockIdx.x;
+    const long long qstep = (long long)gridDim.x * kWaves;
+    for (long long q = q0; q < ngrab; q += qstep) {
+        const long long r0 = grab_row[q], r1 = grab_row[q + 1];
+        for (long long u0 = r0; u0 < r1; u0 += kWave) {
+            const bool in = u0 + lane < r1;
+            const long long d = in ? (long long)(beg[u0 + lane + 1] - beg[u0 + lane]) : 0;
+            ncand += (unsigned)__popcll(__ballot(d >= thr));
+        }
+    }
+    if (lane == 0)
+        cand_s[wave] = ncand;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned all = 0;
+        for (int w = 0; w < kWaves; w++)
+            all += cand_s[w];
+        base_s = all ? atomicAdd(&misc[kCmSources], all) : 0u;
+    }
+    __syncthreads();
+    unsigned slot = base_s;
+    for (int w = 0; w < wave; w++)
+        slot += cand_s[w];
+    for (long long q = q0; q < ngrab; q += qstep) {
         const long long r0 = grab_row[q], r1 = grab_row[q + 1];
       for (long long u0 = r0; u0 < r1; u0 += kWave) {
         const int n = (int)min((long long)kWave, r1 - u0);
         const long long d = lane < n ? (long long)(beg[u0 + lane + 1] - beg[u0 + lane]) : 0;
         unsigned long long cand = __ballot(d >= thr);
-        // a bsrc slot for each candidate row of the group
-        unsigned b0 = 0;
-        if (lane == 0 && cand)
-            b0 = atomicAdd(&misc[3], (unsigned)__popcll(cand));
-        b0 = __builtin_amdgcn_readfirstlane(b0);
         while (cand) {
             const int i = __builtin_ctzll(cand);
-            const unsigned b = b0++;
+            const unsigned b = slot++;
             cand &= cand - 1;
             const long long u = u0 + i;
             const long long lo = (long long)beg[u], hi = (long long)beg[u + 1];
@@ -354,21 +437,23 @@ core_lists_kernel(const OffT *__restrict__ beg, const int32_t *__restrict__ adj,
             for (int k = lane; k < words; k += kWave)
                 seen[k] = 0;
             wave_sync();
-            if (dup || nd == 0 || (long long)b >= nsrc_cap)
+            if ((long long)b >= nsrc_cap)
                 continue;
-            const int parts = (nd + kCorePart - 1) / kCorePart;
-            if (lane < parts) {
-                long long slot;
-                if (parts > 1)
-                    slot = (long long)atomicAdd(&misc[0], 1u);
-                else
-                    slot = cap - 1 - (long long)atomicAdd(&misc[1], 1u);
-                DenseRec<OffT> rc;
-                rc.lo = (OffT)lo;
+            const bool source = !dup && nd > 0;
+            const int parts = source ? (nd + kCorePart - 1) / kCorePart : 0;
+            DenseRec<OffT> rc;
+            rc.lo = (OffT)lo;
+            rc.t0 = 0;
+            rc.t1 = parts == 1 ? nd : 0;
+            rc.b = (int32_t)b;
+            if (lane == 0)
+                recs[cap - 1 - (long long)b] = rc;
+            if (!source)
+                continue;
+            if (parts > 1 && lane < parts) {
                 rc.t0 = lane * kCorePart;
                 rc.t1 = min(nd, (lane + 1) * kCorePart);
-                rc.b = (int32_t)b;
-                recs[slot] = rc;
+                recs[atomicAdd(&misc[kCmLong], 1u)] = rc;
             }
             if (lane == 0)
                 atomicOr(&src_bits[u >> 5], 1u << (u & 31));
@@ -377,11 +462,11 @@ core_lists_kernel(const OffT *__restrict__ beg, const int32_t *__restrict__ adj,
     }
 }
 
-// grab_row[q] = the first row starting at or after entry q 2^kCoreGrabLg
+// grab_row[q] = the first row starting at or after entry q 2^lg
 // (q <= ngrab; grab_row[ngrab] = V).
 template <typename OffT>
 __global__ void __launch_bounds__(kCoreThreads)
-core_grabs_kernel(const OffT *__restrict__ beg, long long V, long long ngrab,
+core_grabs_kernel(const OffT *__restrict__ beg, long long V, long long ngrab, int lg,
                   long long *__restrict__ grab_row)
 {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -391,7 +476,7 @@ core_grabs_kernel(const OffT *__restrict__ beg, long long V, long long ngrab,
         grab_row[q] = V;
         return;
     }
-    const long long at = q << kCoreGrabLg;
+    const long long at = q << lg;
     long long lo = 0, hi = V;  // the first u in [0, V] with beg[u] >= at
     while (lo < hi) {
         const long long mid = (lo + hi) >> 1;
@@ -403,18 +488,19 @@ core_grabs_kernel(const OffT *__restrict__ beg, long long V, long long ngrab,
     grab_row[q] = lo;
 }
 
-// Rows with d+ >= thr (an upper bound on the dense sources), into misc[4].
+// Rows with d+ >= t (an upper bound on the dense sources).
 template <typename OffT>
 __global__ void __launch_bounds__(kCoreThreads)
-core_rows_over_kernel(const OffT *__restrict__ beg, long long V, int thr, unsigned *__restrict__ n)
+core_rows_over_kernel(const OffT *__restrict__ beg, long long V, unsigned *__restrict__ misc)
 {
+    const long long thr = misc[kCmDegree];
     unsigned k = 0;
     for (long long x = (long long)blockIdx.x * blockDim.x + threadIdx.x; x < V;
          x += (long long)gridDim.x * blockDim.x)
         k += (long long)(beg[x + 1] - beg[x]) >= thr;
     k = (unsigned)wave_sum((unsigned long long)k);
     if (lane_id() == 0 && k)
-        atomicAdd(n, k);
+        atomicAdd(misc + kCmOver, k);
 }
 
 // The counting launch.  A wave's item (r, s): u's slice s of B(u) from bsrc
@@ -423,7 +509,7 @@ core_rows_over_kernel(const OffT *__restrict__ beg, long long V, int thr, unsign
 // pieces, wd/4 lanes per target, 64/(wd/4) targets at a time (8 for 32-word
 // slices), kIn per lane in flight.
 template <typename OffT>
-__global__ void __launch_bounds__(kCoreThreads)
+__global__ void __launch_bounds__(kCoreThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
 core_dense_kernel(const DenseRec<OffT> *__restrict__ recs, long long cap,
                   const unsigned *__restrict__ misc_in, unsigned *__restrict__ queues,
                   const uint16_t *__restrict__ pool, const uint32_t *__restrict__ bsrc,
@@ -439,8 +525,8 @@ core_dense_kernel(const DenseRec<OffT> *__restrict__ recs, long long cap,
     const int L = wd >> 2;                            // lanes per target, 4 words each
     const int G = kWave / L;                          // targets per step
     const int g = lane / L, w4 = lane - g * L;        // lanes with g >= G idle
-    const long long n_long = misc_in[0], n_short = misc_in[1];
-    const long long n = n_long + n_short;
+    const unsigned n_long = misc_in[kCmLong];
+    const unsigned n = n_long + misc_in[kCmSources];
     unsigned long long acc = 0;
     // slices in the order: this XCD's (x, x + 8, ...), then the others
     const int x = xcc_id() & (kXcds - 1);
@@ -453,50 +539,62 @@ core_dense_kernel(const DenseRec<OffT> *__restrict__ recs, long long cap,
             if (c % kXcds != x && k-- == 0)
                 return c;
     };
+    // items per grab: a slice's counter takes an atomic every 11.5 ns, which
+    // at one item each bounded the launch (R-MAT 20: 0.48 ms); four grabs per
+    // wave of an XCD still level it
+    const unsigned grab = min(max(n / (4u * (unsigned)gridDim.x * kWaves / kXcds), 1u), 16u);
     int vis = 0, s = slice_at(0);
-    unsigned qn = 0;  // the next item, taken while this one is counted
+    unsigned qn = 0;  // the next grab, taken while this one is counted
     if (lane == 0)
-        qn = atomicAdd(&queues[s * kCoreQueueStride], 1u);
+        qn = atomicAdd(&queues[s * kCoreQueueStride], grab);
     for (;;) {
         const unsigned q = __builtin_amdgcn_readfirstlane(qn);
-        if ((long long)q >= n) {
+        if (q >= n) {
             if (++vis == S)
                 break;
             s = slice_at(vis);
             if (lane == 0)
-                qn = atomicAdd(&queues[s * kCoreQueueStride], 1u);
+                qn = atomicAdd(&queues[s * kCoreQueueStride], grab);
             continue;
         }
-        const long long ri = (long long)q < n_long ? (long long)q : cap - 1 - ((long long)q - n_long);
-        const DenseRec<OffT> rc = recs[ri];
         if (lane == 0)
-            qn = atomicAdd(&queues[s * kCoreQueueStride], 1u);
-        const uint4 bu = ((const uint4 *)(bsrc + (size_t)rc.b * words + (size_t)s * wd))[w4];
-        if (__ballot((bu.x | bu.y | bu.z | bu.w) != 0u) == 0ull)
-            continue;  // no core neighbour of u in this slice
-        const int nt = rc.t1 - rc.t0;
-        const uint16_t *src = pool + (long long)rc.lo + rc.t0;
-        for (int j = lane; j < nt; j += kWave)
-            tg[j] = src[j];
-        wave_sync();
+            qn = atomicAdd(&queues[s * kCoreQueueStride], grab);
+        // the grab's items, one per lane
+        const unsigned qi = min(q + (unsigned)min(lane, (int)grab - 1), n - 1);
+        const DenseRec<OffT> mine =
+            recs[qi < n_long ? (long long)qi : cap - 1 - (long long)(qi - n_long)];
+        const int items = (int)min(grab, n - q);
         const uint4 *base = (const uint4 *)(rows + (size_t)s * Kb * wd) + w4;
-        int t = g < G ? g : nt;
-        for (; t + (kIn - 1) * G < nt; t += kIn * G) {
-            uint4 x[kIn];
+        for (int i = 0; i < items; i++) {
+            const int t0 = readlane(mine.t0, i), nt = readlane(mine.t1, i) - t0;
+            if (nt <= 0)
+                continue;  // not a source, or among the long ones
+            const int b = readlane(mine.b, i);
+            const uint4 bu = ((const uint4 *)(bsrc + (size_t)b * words + (size_t)s * wd))[w4];
+            const uint16_t *src = pool + (long long)readlane(mine.lo, i) + t0;
+            for (int j = lane; j < nt; j += kWave)
+                tg[j] = src[j];
+            if (__ballot((bu.x | bu.y | bu.z | bu.w) != 0u) == 0ull)
+                continue;  // no core neighbour of u in this slice
+            wave_sync();
+            int t = g < G ? g : nt;
+            for (; t + (kIn - 1) * G < nt; t += kIn * G) {
+                uint4 y[kIn];
 #pragma unroll
-            for (int k = 0; k < kIn; k++)
-                x[k] = base[(size_t)tg[t + k * G] * L];
+                for (int k = 0; k < kIn; k++)
+                    y[k] = base[(size_t)tg[t + k * G] * L];
 #pragma unroll
-            for (int k = 0; k < kIn; k++)
-                acc += (unsigned long long)(__popc(x[k].x & bu.x) + __popc(x[k].y & bu.y) +
-                                            __popc(x[k].z & bu.z) + __popc(x[k].w & bu.w));
+                for (int k = 0; k < kIn; k++)
+                    acc += (unsigned long long)(__popc(y[k].x & bu.x) + __popc(y[k].y & bu.y) +
+                                                __popc(y[k].z & bu.z) + __popc(y[k].w & bu.w));
+            }
+            for (; t < nt; t += G) {
+                const uint4 y = base[(size_t)tg[t] * L];
+                acc += (unsigned long long)(__popc(y.x & bu.x) + __popc(y.y & bu.y) +
+                                            __popc(y.z & bu.z) + __popc(y.w & bu.w));
+            }
+            wave_sync();  // before the next item overwrites tg
         }
-        for (; t < nt; t += G) {
-            const uint4 x = base[(size_t)tg[t] * L];
-            acc += (unsigned long long)(__popc(x.x & bu.x) + __popc(x.y & bu.y) +
-                                        __popc(x.z & bu.z) + __popc(x.w & bu.w));
-        }
-        wave_sync();  // before the next item overwrites tg
     }
     acc = wave_sum(acc);
     if (lane == 0 && acc)
@@ -504,6 +602,19 @@ core_dense_kernel(const DenseRec<OffT> *__restrict__ recs, long long cap,
 }
 
 // ------------------------------------------------------------------ host
+// The automatic seed: a power of two near twice the square root of V.  With
+// more, the closure of a smaller graph leaves its top degree class: R-MAT 20
+// closes to 6.2k vertices from 2048, 9.9k from 4096 and 30.5k from 8192
+// (counts of 1.38, 1.60 and 2.39 ms); R-MAT 22 closes to 9.1k from 4096 and
+// from 16384, R-MAT 24 to 12.9k from 4096 up, R-MAT 26 to 17.9k from 16384.
+static int core_auto_seed(long long V)
+{
+    int k = kCoreSeedMin;
+    while (k < kCoreSeedMax && (double)k * (double)k < 4.0 * (double)V)
+        k *= 2;
+    return k;
+}
+
 void core_config(const Ctx *ctx, const trust_params &p, int *K, int *thr, bool *automatic)
 {
     *K = 0;
@@ -511,18 +622,18 @@ void core_config(const Ctx *ctx, const trust_params &p, int *K, int *thr, bool *
     *automatic = false;
     if (p.core_vertices < 0 || p.total_process > 1 || ctx->batch_ngraphs > 0)
         return;
-    const int t = p.core_min_degree > 0 ? p.core_min_degree : kCoreMinDegree;
+    const int low = p.core_min_degree > 0 ? p.core_min_degree : kCoreMinDegreeLow;
     if (p.core_vertices > 0) {
         *K = p.core_vertices;
-    } else if (ctx->g.E >= (1ll << 23) && ctx->g.max_deg >= 2ll * t) {
-        // (a graph without out-degrees of 2t cannot have the heavy tail the
+    } else if (ctx->g.E >= (1ll << 23) && ctx->g.max_deg >= 4ll * low) {
+        // (a graph without such out-degrees cannot have the heavy tail the
         // automatic core asks for below: Chung-Lu 3.8M's fresh count skips
-        // the check, 0.1 ms of its 1.8 ms)
-        *K = kCoreSeedMax;
+        // the check)
+        *K = core_auto_seed(ctx->g.V);
         *automatic = true;
     }
     if (*K)
-        *thr = t;
+        *thr = p.core_min_degree;  // 0: by the core's size
 }
 
 void core_drop(Ctx *ctx)
@@ -548,12 +659,11 @@ static int core_build_t(Ctx *ctx)
     CoreIndex &c = ctx->core;
     const DevCsr &g = ctx->g;
     const long long V = g.V, E = g.E;
-    const int K0 = c.want_K, thr = c.want_thr;
+    const int K0 = c.want_K;
     const OffT *beg = (const OffT *)g.beg.p;
     const int32_t *adj = (const int32_t *)g.adj.p;
     hipStream_t st = ctx->stream;
     c.words = (V + 31) / 32;
-    c.cap = E / std::max(thr, 1) + E / kCorePart + 2;
     int rc;
     if ((rc = c.flag.ensure(sizeof(int) * (size_t)V)) ||
         (rc = c.pos.ensure(sizeof(int) * (size_t)(V + 1))) ||
@@ -566,6 +676,7 @@ static int core_build_t(Ctx *ctx)
         return rc;
     int *flag = (int *)c.flag.p;
     int *din = (int *)c.pos.p;  // the sampled in-counts, until the scan
+    int *list = (int *)c.coreV.p;  // the members as they are found, until the scan
     uint32_t *bits = (uint32_t *)c.bits.p;
     uint32_t *dst_bits = bits, *src_bits = bits + c.words, *dense_cid = bits + 2 * c.words;
     unsigned *misc = (unsigned *)c.misc.p;
@@ -578,76 +689,64 @@ static int core_build_t(Ctx *ctx)
     hipLaunchKernelGGL(core_hist_kernel<OffT>, dim3(blocks), dim3(kCoreThreads), 0, st, beg, V,
                        (const int *)din, (unsigned *)c.hist.p);
     HIPCHK(hipGetLastError());
-    std::vector<unsigned> h(kCoreBins);
-    HIPCHK(hipMemcpyAsync(h.data(), c.hist.p, sizeof(unsigned) * kCoreBins,
-                          hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    // the seed: the top bins, at most k0 vertices, estimates of at least thr
-    const int bmin = core_bin_host(thr);
-    auto seed_cut = [&](long long k0, long long *take) {
-        int bstar = kCoreBins;
-        *take = 0;
-        for (int b = kCoreBins - 1; b >= bmin; b--) {
-            if (*take + h[(size_t)b] > (unsigned long long)k0)
-                break;
-            *take += h[(size_t)b];
-            bstar = b;
-        }
-        return bstar;
-    };
-    long long take = 0;
-    int bstar = seed_cut(K0, &take);
     c.K = K0;
-    c.thr = thr;
     c.built = true;
     c.active = false;
-    // The automatic core needs a heavy tail: its seed's smallest estimates at
-    // least 2t (R-MAT 26: about 12k; a Chung-Lu graph capped at degree 800
-    // has no such vertices, and takes the reference walk anyway)
-    if (take == 0 || (c.want_auto && bstar < core_bin_host(2ll * thr)))
-        return TRUST_OK;
-    // The closure, while it fits; a seed whose closure passes kCoreMax
-    // vertices is halved and closed again (down to kCoreSeedMin), and past
-    // that the seed alone is the core (its targets are whichever lists lie
-    // inside it).
-    const long long xblocks =
-        std::min<long long>((V + kCoreThreads - 1) / kCoreThreads, 8ll * ctx->num_cus);
-    long long members = take;
-    for (long long k0 = K0;;) {
-        hipLaunchKernelGGL(core_seed_kernel<OffT>, dim3(blocks), dim3(kCoreThreads), 0, st, beg,
-                           V, (const int *)din, flag, bstar);
+    // The seed and its closure, while it fits; a seed whose closure passes
+    // kCoreMax vertices is halved and closed again (down to kCoreSeedMin),
+    // and past that the last seed alone is the core (its targets are
+    // whichever lists lie inside it).  All steps are queued at once (a step
+    // with nothing to expand takes 3 us) and the host waits once.
+    const int bmin = core_bin_host(c.want_thr > 0 ? c.want_thr : kCoreMinDegreeLow);
+    unsigned h[kCmLevel];
+    auto close = [&](int k0, int steps) -> int {
+        hipLaunchKernelGGL(core_cut_kernel, dim3(1), dim3(kCoreThreads), 0, st,
+                           (const unsigned *)c.hist.p, bmin, (unsigned)k0, misc);
+        hipLaunchKernelGGL(core_seed_kernel<OffT>, dim3(blocks), dim3(kCoreThreads), 0, st, beg, V,
+                           (const int *)din, flag, list, misc);
+        for (int k = 0; k < steps; k++) {
+            hipLaunchKernelGGL(core_level_kernel, dim3(1), dim3(1), 0, st, misc, k);
+            // (the seed and what it adds are nearly all there is)
+            hipLaunchKernelGGL(core_expand_kernel<OffT>, dim3(k < 2 ? 2 * blocks : blocks / 4),
+                               dim3(kCoreThreads), 0, st, beg, adj, flag, list, misc, k);
+        }
+        hipLaunchKernelGGL(core_degree_kernel, dim3(1), dim3(1), 0, st, misc, c.want_thr);
+        HIPCHK(launch_fill_u32(misc + kCmOver, 0u, 1, st));
+        hipLaunchKernelGGL(core_rows_over_kernel<OffT>, dim3(blocks), dim3(kCoreThreads), 0, st, beg,
+                           V, misc);
         HIPCHK(hipGetLastError());
-        members = take;
-        bool closed = false;
-        for (int step = 0; step < kCoreSteps && !closed && members <= kCoreMax; step++) {
-            HIPCHK(launch_fill_u32(misc + 2, 0u, 1, st));
-            hipLaunchKernelGGL(core_expand_kernel<OffT>, dim3((unsigned)std::max(xblocks, 1ll)),
-                               dim3(kCoreThreads), 0, st, beg, adj, V, flag, misc + 2);
-            hipLaunchKernelGGL(core_promote_kernel, dim3(blocks), dim3(kCoreThreads), 0, st, V,
-                               flag, 0);
-            HIPCHK(hipGetLastError());
-            unsigned added = 0;
-            HIPCHK(hipMemcpyAsync(&added, misc + 2, sizeof(added), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
-            members += added;
-            closed = added == 0;
+        HIPCHK(hipMemcpyAsync(h, misc, sizeof(h), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        return TRUST_OK;
+    };
+    for (int k0 = K0, steps = kCoreSteps;;) {
+        if ((rc = close(k0, steps)))
+            return rc;
+        // The automatic core needs a heavy tail: its seed's smallest
+        // estimates at least 2t (R-MAT 26: about 12k; a Chung-Lu graph capped
+        // at degree 800 has no such vertices, and takes the reference walk
+        // anyway)
+        if (k0 == K0 && steps > 0 &&
+            (h[kCmTake] == 0 ||
+             (c.want_auto && (int)h[kCmCut] < core_bin_host(2ll * (long long)h[kCmDegree]))))
+            return TRUST_OK;
+        if (h[kCmTake] == 0) {  // no smaller seed: the last one alone
+            k0 *= 2;
+            steps = 0;
+            continue;
         }
-        if (members <= kCoreMax)
+        if (h[kCmMembers] <= (unsigned)kCoreMax)
             break;
-        long long t2 = 0;
-        const int b2 = k0 / 2 >= kCoreSeedMin ? seed_cut(k0 / 2, &t2) : kCoreBins;
-        if (t2 == 0) {  // no smaller seed: the seed alone
-            hipLaunchKernelGGL(core_seed_kernel<OffT>, dim3(blocks), dim3(kCoreThreads), 0, st,
-                               beg, V, (const int *)din, flag, bstar);
-            members = take;
-            break;
-        }
-        k0 /= 2;
-        bstar = b2;
-        take = t2;
+        if (k0 / 2 >= kCoreSeedMin)
+            k0 /= 2;
+        else
+            steps = 0;  // the seed alone
     }
-    hipLaunchKernelGGL(core_promote_kernel, dim3(blocks), dim3(kCoreThreads), 0, st, V, flag, 1);
-    HIPCHK(hipGetLastError());
+    const int thr = (int)h[kCmDegree];
+    c.thr = thr;
+    c.cap = E / std::max(thr, 1) + E / kCorePart + 2;
+    c.nsrc_cap = std::max<long long>(h[kCmOver], 1);
+    const unsigned members = h[kCmMembers];
     // bit rows: S slices of wd words, wd a power of two in [4, 32]: a slice
     // row is at most one 128-byte line (a lane reads 16 bytes of it)
     const int nC = (int)members;
@@ -659,19 +758,17 @@ static int core_build_t(Ctx *ctx)
     c.nC = nC;
     c.Kb = Kb;
     c.S = S;
-    // the dense sources' rows B(u): at most one per row with d+ >= thr
-    hipLaunchKernelGGL(core_rows_over_kernel<OffT>, dim3(blocks), dim3(kCoreThreads), 0, st, beg,
-                       V, thr, misc + 4);
-    HIPCHK(hipGetLastError());
-    unsigned over = 0;
-    HIPCHK(hipMemcpyAsync(&over, misc + 4, sizeof(over), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    c.nsrc_cap = std::max<long long>(over, 1);
+    // ranges of entries that the lists kernel's waves take, four per wave
+    const unsigned lblocks = (unsigned)(8 * ctx->num_cus);
+    int grab_lg = 9;
+    while (grab_lg < 20 && (E >> grab_lg) > 16ll * lblocks)
+        grab_lg++;
+    const long long ngrab = (E >> grab_lg) + 1;
     if ((rc = c.rows.ensure((size_t)Kb * (size_t)Kb / 8)) ||
         (rc = c.pool.ensure(sizeof(uint16_t) * (size_t)E)) ||
         (rc = c.recs.ensure(sizeof(DenseRec<OffT>) * (size_t)c.cap)) ||
         (rc = c.bsrc.ensure((size_t)c.nsrc_cap * (size_t)Kb / 8)) ||
-        (rc = c.grabs.ensure(sizeof(long long) * (size_t)((E >> kCoreGrabLg) + 2))))
+        (rc = c.grabs.ensure(sizeof(long long) * (size_t)(ngrab + 1))))
         return rc;
     HIPCHK(launch_scan<int32_t>(flag, nullptr, V, (long long *)ctx->side_bsum.p, (int32_t *)c.pos.p,
                                 st));
@@ -681,11 +778,10 @@ static int core_build_t(Ctx *ctx)
     hipLaunchKernelGGL(core_rows_kernel<OffT>, dim3((unsigned)nC), dim3(kCoreThreads), 0, st, beg,
                        adj, (const int16_t *)c.cid.p, (const int *)c.coreV.p, Kb, S, thr,
                        (uint32_t *)c.rows.p, dst_bits, dense_cid);
-    const long long ngrab = (E >> kCoreGrabLg) + 1;
     hipLaunchKernelGGL(core_grabs_kernel<OffT>,
                        dim3((unsigned)((ngrab + kCoreThreads) / kCoreThreads)), dim3(kCoreThreads),
-                       0, st, beg, V, ngrab, (long long *)c.grabs.p);
-    hipLaunchKernelGGL(core_lists_kernel<OffT>, dim3((unsigned)std::max(xblocks, 1ll)),
+                       0, st, beg, V, ngrab, grab_lg, (long long *)c.grabs.p);
+    hipLaunchKernelGGL(core_lists_kernel<OffT>, dim3(lblocks),
                        dim3(kCoreThreads), 0, st, beg, adj, V, (const int16_t *)c.cid.p,
                        (const uint32_t *)dense_cid, Kb, thr, (uint16_t *)c.pool.p,
                        (DenseRec<OffT> *)c.recs.p, c.cap, (uint32_t *)c.bsrc.p, c.nsrc_cap,
@@ -707,8 +803,8 @@ int core_build(Ctx *ctx)
     if (K < kCoreSeedMin || K > kCoreSeedMax || (K & (K - 1)))
         return fail(TRUST_ERR_ARG, "core_vertices %d: a power of two in [%d, %d]", K,
                     kCoreSeedMin, kCoreSeedMax);
-    if (c.want_thr < 2)
-        return fail(TRUST_ERR_ARG, "core_min_degree %d < 2", c.want_thr);
+    if (c.want_thr < 0 || c.want_thr == 1)
+        return fail(TRUST_ERR_ARG, "core_min_degree %d: 0 or >= 2", c.want_thr);
     return ctx->g.off64 ? core_build_t<int64_t>(ctx) : core_build_t<int32_t>(ctx);
 }
 

@@ -107,7 +107,8 @@ typedef struct trust_params {
      * -1 none, else a power of two in [256, 16384].
      * core_min_degree: 0 automatic (a 48th of the core's vertices, 64 to 384),
      * else >= 2. */
-    int32_t reserved[3];   /* reserved[0]: a tile stream's device tile-cache slots (0: 2n+2) */
+    int32_t reserved[3];   /* reserved[0]: a tile stream's device tile-cache slots (0: every tile
+                              when they take at most 32 GB, else 2n+2) */
     int32_t core_vertices;
     int32_t core_min_degree;
 } trust_params;

@@ -24,8 +24,16 @@ int hip_fail(hipError_t e, const char *what);
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
+    bool borrowed = false;  // a part of another buffer: not freed here
     int ensure(size_t n);
     void release();
+    void borrow(void *q, size_t n)
+    {
+        release();
+        p = q;
+        bytes = n;
+        borrowed = true;
+    }
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;

@@ -61,12 +61,13 @@ int DevBuf::ensure(size_t n)
 
 void DevBuf::release()
 {
-    if (p) {
+    if (p && !borrowed) {
         (void)hipFree(p);
         g_dev_held.fetch_sub(bytes);
     }
     p = nullptr;
     bytes = 0;
+    borrowed = false;
 }
 
 int upload_csr(Ctx *ctx, DevCsr &g, const int64_t *beg, const int32_t *adj, int64_t V, int64_t E,

@@ -106,13 +106,43 @@ int64_t host_max_degree(const int64_t *beg, int64_t V)
 
 void host_parallel_copy(void *dst, const void *src, size_t bytes)
 {
-    constexpr size_t kPiece = 4u << 20;
+    constexpr size_t kPiece = 256u << 10;
     const long long pieces = (long long)((bytes + kPiece - 1) / kPiece);
 #pragma omp parallel for schedule(static)
     for (long long i = 0; i < pieces; i++) {
         const size_t o = (size_t)i * kPiece;
         memcpy((char *)dst + o, (const char *)src + o, std::min(kPiece, bytes - o));
     }
+}
+
+TileFacts host_tile_facts(const trust_csr &c)
+{
+    TileFacts f;
+    f.sound = c.vertices >= 0 && c.edges >= 0 && c.beg && (c.edges == 0 || c.adj) &&
+              c.beg[0] == 0 && c.beg[c.vertices] == c.edges;
+    if (!f.sound)
+        return f;
+    int64_t bad = 0, maxd = 0;
+    int32_t lo = INT32_MAX, hi = -1;
+#pragma omp parallel
+    {
+#pragma omp for schedule(static) reduction(+ : bad) reduction(max : maxd) nowait
+        for (int64_t u = 0; u < c.vertices; u++) {
+            const int64_t d = c.beg[u + 1] - c.beg[u];
+            bad += d < 0;
+            maxd = std::max(maxd, d);
+        }
+#pragma omp for schedule(static) reduction(min : lo) reduction(max : hi)
+        for (int64_t e = 0; e < c.edges; e++) {
+            lo = std::min(lo, c.adj[e]);
+            hi = std::max(hi, c.adj[e]);
+        }
+    }
+    f.sound = bad == 0;
+    f.max_degree = maxd;
+    f.min_id = lo;
+    f.max_id = hi;
+    return f;
 }
 
 void host_tile_row_degrees(const trust_csr *tiles, int n, int c, int64_t rows, int32_t *out)

@@ -35,8 +35,18 @@ int load_folder(const std::string &folder, HostCsr &out);
 // Largest beg[u+1]-beg[u] (OpenMP, host).
 int64_t host_max_degree(const int64_t *beg, int64_t V);
 
-// memcpy with all OpenMP threads, in 4 MB pieces.
+// memcpy with all OpenMP threads, in 256 KB pieces.
 void host_parallel_copy(void *dst, const void *src, size_t bytes);
+
+// One pass over a tile (all OpenMP threads): offsets that span its entries and
+// never decrease (sound; the rest only then), its longest row and its ids'
+// range (min_id INT32_MAX and max_id -1 without entries).
+struct TileFacts {
+    bool sound = false;
+    int64_t max_degree = 0;
+    int32_t min_id = 0, max_id = -1;
+};
+TileFacts host_tile_facts(const trust_csr &c);
 
 // Row sums of tile class c of an n x n partition (tiles[c*n + b], b < n):
 // the global out-degree of each of its `rows` vertices, saturated to int32.

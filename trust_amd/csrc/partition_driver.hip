@@ -115,7 +115,6 @@ static int upload_pinned(Ctx *ctx, PinnedStage &st, DevCsr &g, const trust_csr &
     g.V = t.vertices;
     g.E = t.edges;
     g.off64 = off64;
-    g.max_deg = host_max_degree(t.beg, t.vertices);
     if (ab > 0)
         HIPCHK(hipMemcpyAsync(g.adj.p, h, ab, hipMemcpyHostToDevice, s));
     if (off64) {
@@ -241,6 +240,8 @@ static int journal_add(Journal &jr, long long id, int n, unsigned long long c, u
 }
 
 // Streams all jobs of an n x n partition; tiles[i*n+j] is tile (i,j).
+// cache_slots: tiles held on the device (0: all of them when they are small,
+// else 2n + 2, enough to prefetch).
 // job_counts (nullable, n^3 entries) receives each job's count.  With a
 // journal path, jobs already in the journal are skipped and each new job is
 // appended as its count lands; max_new_jobs > 0 stops after that many new
@@ -255,49 +256,82 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
     int64_t maxd = 0, Vsum = 0, Esum = 0;
     for (int t = 0; t < n * n; t++) {
         off64 = off64 || tiles[t].edges >= kMaxEdges32;
-        for (int64_t u = 0; u < tiles[t].vertices; u++)
-            maxd = std::max(maxd, tiles[t].beg[u + 1] - tiles[t].beg[u]);
         Esum += tiles[t].edges;
     }
     for (int i = 0; i < n; i++)
         Vsum += tiles[(size_t)i * n].vertices;
+    // Each tile is read once (the ids only when they are checked): checking
+    // the three tiles of every job read each of them 3n times, 60 of the
+    // 140 ms of R-MAT 20 in 4 x 4 tiles.
+    const bool validate = !(p.flags & TRUST_FLAG_NO_VALIDATE);
+    int64_t ids = int64_t(1) << 31;  // hash and probe ids are below this
+    if (validate) {
+        std::vector<TileFacts> facts((size_t)n * n);
+        bool good = true;
+        int32_t top = -1;
+        for (int t = 0; t < n * n && good; t++) {
+            facts[t] = host_tile_facts(tiles[t]);
+            good = facts[t].sound && facts[t].min_id >= 0 &&
+                   tiles[t].vertices == tiles[t / n * n].vertices;
+            maxd = std::max(maxd, facts[t].max_degree);
+            top = std::max(top, facts[t].max_id);
+        }
+        for (int t = 0; t < n * n && good; t++)  // walk ids of (i,k) are rows of every (k,j)
+            good = facts[t].max_id < tiles[(size_t)(t % n) * n].vertices;
+        ids = (int64_t)top + 1;
+        if (!good) {  // the first bad tile of the first bad job
+            for (int i = 0; i < n; i++)
+                for (int j = 0; j < n; j++)
+                    for (int k = 0; k < n; k++)
+                        if (int rc = check_job_tiles(tiles[i * n + j], tiles[i * n + k], tiles[k * n + j]))
+                            return rc;
+            return fail(TRUST_ERR_FORMAT, "inconsistent tiles");
+        }
+    } else {
+        for (int t = 0; t < n * n; t++)
+            maxd = std::max(maxd, host_max_degree(tiles[t].beg, tiles[t].vertices));
+    }
     if (maxd > (int64_t)(INT32_MAX / 64))
         return fail(TRUST_ERR_OVERFLOW, "tile degree %lld too large", (long long)maxd);
-    if (!(p.flags & TRUST_FLAG_NO_VALIDATE))
-        for (int i = 0; i < n; i++)
-            for (int j = 0; j < n; j++)
-                for (int k = 0; k < n; k++) {
-                    int rc = check_job_tiles(tiles[i * n + j], tiles[i * n + k], tiles[k * n + j]);
-                    if (rc)
-                        return rc;
-                }
     LaunchPlan L;
     int rc = resolve_launch(ctx, p, maxd, Vsum, off64, L);
     if (rc)
         return rc;
-    cache_slots = std::max(3, std::min(cache_slots, n * n));
-    std::vector<TileSlot> slots((size_t)cache_slots);
-    for (auto &s : slots) {
-        HIPCHK(hipEventCreateWithFlags(&s.ready, hipEventDisableTiming));
-        HIPCHK(hipEventCreateWithFlags(&s.released, hipEventDisableTiming));
-    }
-    // Size every device buffer for the largest tile up front: a buffer is
-    // never reallocated while a queued copy or count may still use it.
     int64_t maxV = 0, maxE = 0;
     for (int t = 0; t < n * n; t++) {
         maxV = std::max(maxV, tiles[t].vertices);
         maxE = std::max(maxE, tiles[t].edges);
     }
+    // Every device buffer is sized for the largest tile up front: none is
+    // reallocated while a queued copy or count may still use it.  The slots
+    // are parts of one allocation.
+    const size_t beg_bytes = ((off64 ? 8 : 4) * (size_t)(maxV + 1) + 255) & ~(size_t)255;
+    const size_t adj_bytes = (sizeof(int32_t) * (size_t)std::max<int64_t>(maxE, 1) + 255) & ~(size_t)255;
+    // Unless the caller chose, all tiles stay when they take at most 32 GB
+    // of the 288: each is then copied once, not once for every row of jobs.
+    const size_t slot_bytes = beg_bytes + adj_bytes;
+    const bool keep_all = cache_slots <= 0 && slot_bytes * (size_t)n * (size_t)n <= (32ull << 30);
+    const int few = std::max(3, std::min(cache_slots > 0 ? cache_slots : 2 * n + 2, n * n));
+    cache_slots = keep_all ? std::max(3, n * n) : few;
+    DevBuf slab;
+    rc = slab.ensure(slot_bytes * (size_t)cache_slots);
+    if (rc == TRUST_ERR_OOM && cache_slots > few) {
+        cache_slots = few;
+        rc = slab.ensure(slot_bytes * (size_t)cache_slots);
+    }
+    if (rc)
+        return rc;
+    std::vector<TileSlot> slots((size_t)cache_slots);
+    for (size_t q = 0; q < slots.size(); q++) {
+        TileSlot &s = slots[q];
+        HIPCHK(hipEventCreateWithFlags(&s.ready, hipEventDisableTiming));
+        HIPCHK(hipEventCreateWithFlags(&s.released, hipEventDisableTiming));
+        s.g.beg.borrow((char *)slab.p + q * slot_bytes, beg_bytes);
+        s.g.adj.borrow((char *)slab.p + q * slot_bytes + beg_bytes, adj_bytes);
+    }
     rc = ctx->staging.ensure(sizeof(int64_t) * (size_t)(maxV + 1));
     if (rc)
         return rc;
-    for (auto &s : slots) {
-        rc = s.g.beg.ensure((off64 ? 8 : 4) * (size_t)(maxV + 1));
-        if (!rc)
-            rc = s.g.adj.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(maxE, 1));
-        if (rc)
-            return rc;
-    }
     // uploads go through two pinned buffers, each sized for the largest tile
     PinnedStage stage;
     const size_t stage_bytes = ((sizeof(int32_t) * (size_t)maxE + 255) & ~(size_t)255) +
@@ -338,6 +372,17 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
     DevBuf degs;
     std::vector<TileWalk> walks(short_walk ? (size_t)n : 0);
     std::vector<int> walk_row(walks.size(), -1);  // the tile row i each walk was built for
+    if (short_walk && keep_all) {
+        // the walks' buffers for the largest tile at once: growing one frees
+        // it, which waits for the device (without room they are sized as
+        // they are needed)
+        const size_t ob = off64 ? 8 : 4, most = sizeof(int32_t) * (size_t)std::max<int64_t>(maxE, 1);
+        bool room = !ctx->wi.recs.ensure(2 * most) && !ctx->wi.rel.ensure(most) &&
+                    !ctx->side_cnt.ensure(2 * sizeof(int) * (size_t)std::max<int64_t>(maxV, 1));
+        for (TileWalk &w : walks)
+            room = room && !w.out_ids.ensure(most) && !w.in_ids.ensure(most) &&
+                   !w.out_beg.ensure(ob * (size_t)(maxV + 1)) && !w.in_beg.ensure(ob * (size_t)(maxV + 1));
+    }
     if (short_walk) {
         // global out-degree of every vertex, class by class (sum over its tile row)
         std::vector<int32_t> d((size_t)deg_off[n]);
@@ -540,11 +585,13 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
             CsrViews vo{th.beg.p, (const int32_t *)th.adj.p, w.out_beg.p,
                         (const int32_t *)w.out_ids.p, tp.beg.p, (const int32_t *)tp.adj.p};
             vo.entries = w.x_out;
+            vo.ids = ids;
             if ((rc = count_view(vo, rows_of[ji], (TcCtl *)ctls.p + 2 * job)))
                 return rc;
             CsrViews vi{tp.beg.p, (const int32_t *)tp.adj.p, w.in_beg.p,
                         (const int32_t *)w.in_ids.p, th.beg.p, (const int32_t *)th.adj.p};
             vi.entries = w.x_in;
+            vi.ids = ids;
             if ((rc = count_view(vi, rows_of[jk], (TcCtl *)ctls.p + 2 * job + 1)))
                 return rc;
         } else {
@@ -552,6 +599,7 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
             CsrViews v{th.beg.p, (const int32_t *)th.adj.p, tw.beg.p, (const int32_t *)tw.adj.p,
                        tp.beg.p, (const int32_t *)tp.adj.p};
             v.entries = tw.E;
+            v.ids = ids;
             if ((rc = count_view(v, tiles[cur[0]].vertices, (TcCtl *)ctls.p + job)))
                 return rc;
         }
@@ -676,9 +724,7 @@ extern "C" int trust_count_tiles(const trust_csr *tiles, int n, const trust_para
     rc = ctx_init(&ctx, p->device);
     if (rc)
         return rc;
-    // reserved[0]: device tile-cache slots (0 = 2n+2, enough to prefetch)
-    int slots = p->reserved[0] > 0 ? p->reserved[0] : 2 * n + 2;
-    return stream_tiles(&ctx, tiles, n, *p, slots, nullptr, r);
+    return stream_tiles(&ctx, tiles, n, *p, p->reserved[0], nullptr, r);
 }
 
 extern "C" int trust_count_tiles_journal(const trust_csr *tiles, int n, const trust_params *p,
@@ -694,9 +740,8 @@ extern "C" int trust_count_tiles_journal(const trust_csr *tiles, int n, const tr
     rc = ctx_init(&ctx, p->device);
     if (rc)
         return rc;
-    int slots = p->reserved[0] > 0 ? p->reserved[0] : 2 * n + 2;
     long long remaining = 0;
-    rc = stream_tiles(&ctx, tiles, n, *p, slots, job_counts, r, journal, (long long)max_new_jobs,
+    rc = stream_tiles(&ctx, tiles, n, *p, p->reserved[0], job_counts, r, journal, (long long)max_new_jobs,
                       &remaining);
     if (rc)
         return rc;

@@ -273,11 +273,11 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
                   bool preplanned, hipStream_t s, hipEvent_t ev_plan, hipEvent_t ev_count,
                   const SegView *seg, bool plan_only, bool with_core)
 {
-    int rc = ctx->list.ensure(sizeof(int32_t) * (size_t)(V + kMaxExtra));
-    if (rc)
-        return rc;
-    rc = ctx->block_counts.ensure(kPlanScratch);
-    if (rc)
+    // a list made elsewhere is in place already: growing the buffer here would
+    // drop it
+    int rc = TRUST_OK;
+    if (!preplanned && ((rc = ctx->list.ensure(sizeof(int32_t) * (size_t)(V + kMaxExtra))) ||
+                        (rc = ctx->block_counts.ensure(kPlanScratch))))
         return rc;
     // a list made elsewhere, and the instrumented mode's per-vertex outputs,
     // know whole vertices only

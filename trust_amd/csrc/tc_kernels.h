@@ -258,18 +258,22 @@ __host__ __device__ inline int group_parts(int dW, int part_entries, int tier)
     return dW > e ? (dW + e - 1) / e : 1;
 }
 
-// Parts of the wave tier.  In a graph of less than 2 M walk entries the waves
-// that take a vertex of some 50 to 100 neighbours are the last to end, by
-// 150 us at R-MAT 16.  There a vertex fills a list position per `each` walk
-// entries, about a 32768th of the walk (a quarter of a wave's share) and 16
-// at least.  The position holds the part's number above kPartShift bits of
-// the vertex, so a vertex has at most kMaxWaveParts.
+// Parts of the wave tier.  In a graph of up to some ten million walk entries
+// the waves that take a vertex of 30 to 100 neighbours are the last to end
+// (R-MAT 16: by 150 us of 240).  There a vertex fills a list position per
+// `each` walk entries, a 131072nd of the walk (16 parts per wave) and 16 at
+// least; the parts beyond the first stand before the tier's vertices and are
+// chunks of their own.  From 13 M entries on `each` passes the degree that
+// sends a vertex to a workgroup.  Counts with whole vertices, with parts:
+// R-MAT 16 241, 155 us; R-MAT 18 775, 570 us; R-MAT 19 1650, 1080 us.
+// The position holds the part's number above kPartShift bits of the vertex,
+// so a vertex has at most kMaxWaveParts.
 constexpr int kPartShift = 26;
 constexpr int kMaxWaveParts = 32;
-constexpr long long kWaveExtra = 32768;
+constexpr long long kWaveExtra = 131072;
 inline int walk_wave_part(long long walk_entries, long long V)
 {
-    if (walk_entries <= 0 || walk_entries >= (2 << 20) || V > (1 << kPartShift))
+    if (walk_entries <= 0 || walk_entries >= (8 << 20) || V > (1 << kPartShift))
         return 0;
     const long long e = (walk_entries + kWaveExtra - 1) / kWaveExtra;
     return e < 16 ? 16 : (int)e;

@@ -1149,13 +1149,29 @@ tc_count_kernel(TcArgs<OffT>)
         // With no more chunks than waves, wave w takes chunk w and no
         // counter is touched; consecutive chunks go to different workgroups
         // (the list's first chunks are its heaviest).
+        // The tier's list holds the parts beyond a vertex's first (wave_parts),
+        // each a chunk of its own, then every vertex (its first part).
         const long long items = a->ctl->list_begin[kTierWave + 1] - a->ctl->list_begin[kTierWave];
-        // chosen here: at least two grabs per wave, at most 64 vertices each
-        // (larger chunks of a skewed list leave long ones for the end)
-        int chunk = a->chunk_wave;
-        if (chunk <= 0)
-            chunk = a->wave_part ? 1 : max(1, min(kWave, (int)(items / (2ll * gridDim.x * nwaves))));
-        const unsigned int n = rank_chunks(items, chunk, a->rank, a->nranks);
+        const unsigned int extra = (unsigned int)a->ctl->extra[kTierWave];
+        const unsigned int whole = (unsigned int)items - extra;
+        const unsigned int waves = gridDim.x * (unsigned int)nwaves;
+        // chosen here: two grabs per wave at least, of at most 64 vertices; but
+        // four per wave from the first quarter, since lists come in descending
+        // length.  With a quarter's chunks as large as the others', the waves
+        // that took 10 to 64 of the longest at once ended last: R-MAT 18
+        // 775 us, now 570; R-MAT 22 with int64 offsets 2.65 ms, now 2.22.
+        // Single vertices all along cost what packs give (Chung-Lu, 3.8 M
+        // vertices: 450 us, 1040).  A batch's list comes graph by graph.
+        unsigned int chunk = a->chunk_wave, fchunk = 1, fronts = 0;
+        if (a->chunk_wave <= 0) {
+            chunk = kMode == kModeBatch ? whole : whole - whole / 4;
+            chunk = max(1u, min((unsigned int)kWave, chunk / (2u * waves)));
+            fchunk = max(1u, min(chunk, whole / (16u * waves)));
+            fronts = kMode == kModeBatch ? 0 : whole / (4u * fchunk);
+        }
+        const unsigned int front = extra + fronts * fchunk;  // where the others begin
+        const unsigned int n = rank_chunks(
+            extra + fronts + ((unsigned int)items - front + chunk - 1u) / chunk, 1, a->rank, a->nranks);
         constexpr bool kBatch = kMode == kModeBatch;
         constexpr int kShards = kBatch ? kXcds : kWaveShards;
         const bool fixed = !kBatch && n <= gridDim.x * (unsigned int)nwaves;
@@ -1167,8 +1183,17 @@ tc_count_kernel(TcArgs<OffT>)
             if (j >= n)
                 break;
             const long long lb = a->ctl->list_begin[kTierWave], le = a->ctl->list_begin[kTierWave + 1];
-            const long long first = lb + ((long long)j * a->nranks + a->rank) * chunk;
-            const long long last = min(first + (long long)chunk, le);
+            const unsigned int c = j * (unsigned int)a->nranks + (unsigned int)a->rank;
+            unsigned int at = c, step = 1;
+            if (c >= extra + fronts) {
+                at = front + (c - extra - fronts) * chunk;
+                step = chunk;
+            } else if (c >= extra) {
+                at = extra + (c - extra) * fchunk;
+                step = fchunk;
+            }
+            const long long first = lb + at;
+            const long long last = min(first + (long long)step, le);
             for (long long i = first; i < last;)
                 i += wave_next<OffT, kMode, kU>(a, i, last, wtab, mark, sum);
         } while (!fixed);
@@ -1254,19 +1279,26 @@ __global__ void __launch_bounds__(1024) plan_count_kernel(PlanArgs<OffT> p)
 }
 
 template <typename OffT>
-__global__ void __launch_bounds__(1024) plan_scatter_kernel(PlanArgs<OffT> p, int nblocks)
+// Above 80 SGPRs a CU holds one workgroup of 1024 threads instead of two
+// (3.8 M vertices: 48 us, 30).
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80)))
+plan_scatter_kernel(PlanArgs<OffT> p, int nblocks)
 {
-    __shared__ int all[2 * kNumTiers], before[kNumTiers];
-    __shared__ int wcount[kNumTiers][1024 / kWave];
-    __shared__ int run[kNumTiers];
+    // index kNumTiers: the wave tier's parts beyond a vertex's first, which
+    // come before its vertices
+    constexpr int kRuns = kNumTiers + 1;
+    __shared__ int all[2 * kNumTiers], before[kRuns];
+    constexpr int kRow = 1024 / kWave;  // most waves in the workgroup
+    __shared__ int wcount[kRuns][kRow];
+    __shared__ int run[kRuns];
     const int wave = threadIdx.x / kWave, nwaves = blockDim.x / kWave;
     if (threadIdx.x < 2 * kNumTiers)
         all[threadIdx.x] = 0;
-    if (threadIdx.x < kNumTiers)
+    if (threadIdx.x < kRuns)
         before[threadIdx.x] = 0;
     __syncthreads();
     {
-        int sum[2 * kNumTiers] = {0}, mine[kNumTiers] = {0};
+        int sum[2 * kNumTiers] = {0}, mine[kRuns] = {0};
         for (int b = threadIdx.x; b < nblocks; b += blockDim.x) {
             const int4 c = ((const int4 *)p.block_counts)[2 * b];
             const int4 e = ((const int4 *)p.block_counts)[2 * b + 1];
@@ -1275,15 +1307,17 @@ __global__ void __launch_bounds__(1024) plan_scatter_kernel(PlanArgs<OffT> p, in
             for (int q = 0; q < 2 * kNumTiers; q++) {
                 sum[q] += v[q];
                 if (q < kNumTiers && b < (int)blockIdx.x)
-                    mine[q] += v[q];
+                    mine[q] += q == kTierWave ? v[q] - v[kNumTiers + q] : v[q];
             }
+            if (b < (int)blockIdx.x)
+                mine[kNumTiers] += v[kNumTiers + kTierWave];
         }
 #pragma unroll
         for (int q = 0; q < 2 * kNumTiers; q++) {
             const int x = wave_total(sum[q]);
             if (lane_id() == 0 && x)
                 atomicAdd(&all[q], x);
-            if (q < kNumTiers) {
+            if (q < kRuns) {
                 const int y = wave_total(mine[q]);
                 if (lane_id() == 0 && y)
                     atomicAdd(&before[q], y);
@@ -1295,7 +1329,12 @@ __global__ void __launch_bounds__(1024) plan_scatter_kernel(PlanArgs<OffT> p, in
         int base = 0;
         for (int q = 0; q < (int)threadIdx.x; q++)
             base += all[q];
-        run[threadIdx.x] = base + before[threadIdx.x];
+        if (threadIdx.x == kTierWave) {
+            run[kNumTiers] = base + before[kNumTiers];
+            run[kTierWave] = base + all[kNumTiers + kTierWave] + before[kTierWave];
+        } else {
+            run[threadIdx.x] = base + before[threadIdx.x];
+        }
         if (blockIdx.x == 0) {
             p.ctl->list_begin[threadIdx.x] = base;
             p.ctl->extra[threadIdx.x] = all[kNumTiers + threadIdx.x];
@@ -1311,38 +1350,60 @@ __global__ void __launch_bounds__(1024) plan_scatter_kernel(PlanArgs<OffT> p, in
         int parts = 1;
         const int tier = u < hi ? plan_tier(p, u, parts) : kTierNone;
         const bool split = __ballot(parts > 1) != 0;
-        int pos = 0;  // in the wave, within the tier
+        int pos = 0, more = 0;  // in the wave, within the tier (more: of the extra parts)
+        // a vertex's positions lie side by side, but in the wave tier its
+        // first stands among the vertices and the rest among the extras
+        const int put = tier == kTierWave ? 1 : parts;
 #pragma unroll
         for (int t = 0; t < kNumTiers; t++) {
             int total, at;
-            if (split) {
-                const int x = tier == t ? parts : 0, incl = wave_scan_add(x);
-                total = readlane(incl, kWave - 1);
-                at = incl - x;
-            } else {
+            if (!split || t == kTierWave) {
                 const unsigned long long m = __ballot(tier == t);
                 total = __popcll(m);
                 at = __builtin_amdgcn_mbcnt_hi((unsigned int)(m >> 32),
                                                __builtin_amdgcn_mbcnt_lo((unsigned int)m, 0));
+            } else {
+                const int x = tier == t ? put : 0;
+                const int incl = wave_scan_add(x);
+                total = readlane(incl, kWave - 1);
+                at = incl - x;
             }
+            pos = tier == t ? at : pos;
             if (lane_id() == 0)
                 wcount[t][wave] = total;
-            pos = tier == t ? at : pos;
+        }
+        if (p.wave_part) {
+            const int x = tier == kTierWave ? parts - 1 : 0;
+            const int incl = split ? wave_scan_add(x) : 0;
+            more = incl - x;
+            if (lane_id() == kWave - 1)
+                wcount[kNumTiers][wave] = incl;
+        }
+        __syncthreads();
+        if (threadIdx.x < kRuns * kRow) {  // a wave's first position, per tier
+            const int t = threadIdx.x / kRow, w = threadIdx.x % kRow;
+            const int x = w < nwaves && (t < kNumTiers || p.wave_part) ? wcount[t][w] : 0;
+            int incl = x;
+#pragma unroll
+            for (int d = 1; d < kRow; d *= 2) {
+                const int y = __shfl_up(incl, d, kRow);
+                incl += w >= d ? y : 0;
+            }
+            const int at = run[t] + incl;
+            wcount[t][w] = at - x;
+            if (w == kRow - 1)
+                run[t] = at;
         }
         __syncthreads();
         if (tier < kNumTiers) {
-            pos += run[tier];
-            for (int w = 0; w < wave; w++)
-                pos += wcount[tier][w];
-            for (int q = 0; q < parts; q++)
-                p.list[pos + q] = tier == kTierWave ? (int32_t)u | q << kPartShift : (int32_t)u;
-        }
-        __syncthreads();
-        if (threadIdx.x < kNumTiers) {
-            int sum = 0;
-            for (int w = 0; w < nwaves; w++)
-                sum += wcount[threadIdx.x][w];
-            run[threadIdx.x] += sum;
+            pos += wcount[tier][wave];
+            for (int q = 0; q < put; q++)
+                p.list[pos + q] = (int32_t)u;
+            if (put < parts) {
+                more += wcount[kNumTiers][wave];
+                for (int q = 1; q < parts; q++)
+                    p.list[more + q - 1] = (int32_t)u | q << kPartShift;
+            }
         }
         __syncthreads();
     }

@@ -615,6 +615,22 @@ static int core_auto_seed(long long V)
     return k;
 }
 
+// The automatic core's sizes.  It needs lists that meet often and a count
+// that its build (300 us at R-MAT 20) does not outweigh.  Index and count
+// without and with the core: R-MAT 20, 8.5 M edges of 0.55 M vertices (15 to
+// one) 1.35, 1.75 ms; 10.5 M (18) 1.68, 1.53 ms; R-MAT 21, 14 M (14) 1.90,
+// 2.03 ms; R-MAT 22, 20 M (11.7) 2.5, 3.1 ms; R-MAT 23, 33 M (10.6) 3.6, 4.0
+// ms, 41 M (12.3) 6.1, 5.0 ms; R-MAT 24, 66 M (11.2) 8.0, 7.7 ms.  A context
+// that counts once also pays 2 ms for the buffers: R-MAT 20, 16 M 8.6, 10.5
+// ms; R-MAT 21, 47 M 24.3, 19.9 ms.
+static bool core_pays(const Ctx *ctx)
+{
+    const long long V = ctx->g.V, E = ctx->g.E;
+    if (ctx->counts_once)
+        return E >= 24ll << 20 && E >= 16 * V;
+    return E >= 9ll << 20 && E >= (E < 32ll << 20 ? 14 : 11) * V;
+}
+
 void core_config(const Ctx *ctx, const trust_params &p, int *K, int *thr, bool *automatic)
 {
     *K = 0;
@@ -625,7 +641,7 @@ void core_config(const Ctx *ctx, const trust_params &p, int *K, int *thr, bool *
     const int low = p.core_min_degree > 0 ? p.core_min_degree : kCoreMinDegreeLow;
     if (p.core_vertices > 0) {
         *K = p.core_vertices;
-    } else if (ctx->g.E >= (1ll << 23) && ctx->g.max_deg >= 4ll * low) {
+    } else if (core_pays(ctx) && ctx->g.max_deg >= 4ll * low) {
         // (a graph without such out-degrees cannot have the heavy tail the
         // automatic core asks for below: Chung-Lu 3.8M's fresh count skips
         // the check)

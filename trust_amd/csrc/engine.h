@@ -176,6 +176,7 @@ struct CoreIndex {
 struct Ctx {
     int device = 0;
     bool ready = false;
+    bool counts_once = false;  // the context ends with its first count
     hipStream_t stream = nullptr;
     hipStream_t copy_stream = nullptr;
     // the large-LDS launch runs here, beside the main launch (fork / join)
@@ -301,7 +302,9 @@ void core_drop(Ctx *ctx);
 void core_release(Ctx *ctx);
 // A graph whose top out-degree is under 24 times the mean takes the
 // reference walk on every family measured (R-MAT 10-18, Chung-Lu, ER, BA:
-// 1.8 to 19 times; R-MAT 20 and up, which take the short side: 27 and up).
+// 1.8 to 19 times; R-MAT 20 and up, which take the short side: 27 and up);
+// where the dense core is wanted the line is 12 times, since with it dense
+// R-MAT graphs (12 to 23 times) take the short side.
 // Only the order of the passes follows from it: reference_pass yields the
 // probe totals that decide, and with `starts` the reference walk's start
 // index (ctx->ref_built) unless there is no room for it.

@@ -509,7 +509,11 @@ static int prepare_side(Ctx *ctx, bool force, bool starts, ResidentRun &R)
             ctx->side_stats_ready = true;
         }
     }
-    R.side = force || (double)ctx->side_w_short <= kShortWalkShare * (double)ctx->side_w_ref;
+    // (of the short walk's probes those that the dense core takes over do not
+    // count)
+    const uint64_t core_probes = ctx->core.active ? ctx->core.dense_probes : 0;
+    R.side = force ||
+             (double)(ctx->side_w_short - core_probes) <= kShortWalkShare * (double)ctx->side_w_ref;
     if (R.side && !ctx->side_built) {
         if (made_starts) {  // the short side after all
             HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -1062,6 +1066,7 @@ extern "C" int trust_count_csr(const int64_t *beg, const int32_t *adj, int64_t V
     if (!p)
         return fail(TRUST_ERR_ARG, "null params");
     Ctx ctx;
+    ctx.counts_once = true;
     int rc = ctx_init(&ctx, p->device);
     if (rc)
         return rc;
@@ -1088,6 +1093,7 @@ extern "C" int trust_triangle_count(int rank, const char *folder, int total_proc
     p.blocks = blocks > 0 ? blocks : 0;
     p.chunk = chunk_size > 0 ? chunk_size : 0;
     Ctx ctx;
+    ctx.counts_once = true;
     rc = ctx_init(&ctx, 0);
     if (rc)
         return rc;

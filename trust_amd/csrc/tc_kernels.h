@@ -226,7 +226,12 @@ hipError_t launch_side_stats(const OffT *beg, const int32_t *adj, long long V,
                              unsigned long long *stats, hipStream_t stream);
 // The short-side walk is chosen by default when it makes at most this share
 // of the reference walk's probes (its lists are shorter, so a probe costs
-// more; measured break-even near 0.45-0.5 on R-MAT).
+// more; measured break-even near 0.45-0.5 on R-MAT).  Probes that the dense
+// core takes over cost next to nothing and are left out of the share: on
+// R-MAT graphs of 20 to 80 pairs per vertex they are two thirds of the walk.
+// Index and count by the reference walk, by the short one with its core:
+// scale 19, 32 pairs per vertex 3.25, 1.81 ms; scale 20, 22 pairs 4.56, 2.37
+// ms; 80 pairs 38.5, 11.1 ms; scale 18, 48 pairs 2.47, 1.58 ms.
 constexpr double kShortWalkShare = 0.45;
 
 // Parts of the workgroup tiers.  One vertex's walk can hold a good share of a

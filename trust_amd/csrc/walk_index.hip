@@ -825,7 +825,8 @@ static int ref_pass(Ctx *ctx, WalkEntry<OffT> *ent, unsigned long long *stats_ou
 bool walk_probably_reference(const Ctx *ctx)
 {
     const DevCsr &g = ctx->g;
-    return (double)g.max_deg * (double)g.V < 24.0 * (double)g.E;
+    const double share = ctx->core.want_K ? 12.0 : 24.0;
+    return (double)g.max_deg * (double)g.V < share * (double)g.E;
 }
 
 int reference_pass(Ctx *ctx, bool starts)

@@ -13,12 +13,12 @@ import trust_amd as T
 pytestmark = pytest.mark.gpu
 
 
-def rows_graph(n, seed):
-    """n rows in descending length (2 to 60) over n + 70 later ids."""
+def rows_graph(n, longest, seed):
+    """n rows in descending length (2 to longest) over n + 130 later ids."""
     rng = np.random.default_rng(seed)
-    m = n + 70
-    deg = np.maximum(2, 60 - 58 * np.arange(n) // max(n // 2, 1))
-    lists = [np.sort(i + 1 + rng.permutation(min(m - i - 1, 90))[:d]) for i, d in enumerate(deg)]
+    m = n + 130
+    deg = np.maximum(2, longest - (longest - 2) * np.arange(n) // max(n // 2, 1))
+    lists = [np.sort(i + 1 + rng.permutation(min(m - i - 1, 120))[:d]) for i, d in enumerate(deg)]
     lists += [np.zeros(0, np.int64)] * (m - n)
     beg = np.concatenate([[0], np.cumsum([len(x) for x in lists])])
     adj = np.concatenate(lists).astype(np.int32)
@@ -27,9 +27,10 @@ def rows_graph(n, seed):
 
 
 @pytest.mark.parametrize("n", [1, 3, 4, 31, 32, 33, 127, 128, 129, 255, 257, 1023, 1025, 4099])
-def test_chunks_match_oracle(gpu, n):
-    print(f"[gpu] wave chunks {n}", flush=True)
-    beg, adj = rows_graph(n, n)
+@pytest.mark.parametrize("longest", [64, 65, 100])  # to 64: all chunks alike
+def test_chunks_match_oracle(gpu, n, longest):
+    print(f"[gpu] wave chunks {n} {longest}", flush=True)
+    beg, adj = rows_graph(n, longest, n)
     want = oracle.count_merge(beg, adj)
     for load in (0, T.FLAG_OFFSETS64):
         with T.Context(gpu) as c:

@@ -124,7 +124,7 @@ struct TcArgs {
     int wave_slots;          // LDS ints per wave table
     int wave_lg;
     int chunk_group;         // vertices per grab, spill/group tiers
-    int chunk_wave;          // vertices per grab, wave tier (0: chosen by the kernel)
+    int chunk_wave;          // vertices per grab, wave tier (0: chosen by the kernel, -1: all alike)
     int part_entries;        // walk entries of a workgroup-tier part (0: vertices are whole)
     int wave_part;           // walk entries of a wave-tier part (0: vertices are whole)
     int pack_rows;           // rows a pack of the wave tier may hold (0, 1: no packs)

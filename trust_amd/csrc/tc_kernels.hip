@@ -1152,7 +1152,8 @@ tc_count_kernel(TcArgs<OffT>)
         // The tier's list holds the parts beyond a vertex's first (wave_parts),
         // each a chunk of its own, then every vertex (its first part).
         const long long items = a->ctl->list_begin[kTierWave + 1] - a->ctl->list_begin[kTierWave];
-        const unsigned int extra = (unsigned int)a->ctl->extra[kTierWave];
+        constexpr bool kBatch = kMode == kModeBatch;  // whole vertices, chunks alike
+        const unsigned int extra = kBatch ? 0u : (unsigned int)a->ctl->extra[kTierWave];
         const unsigned int whole = (unsigned int)items - extra;
         const unsigned int waves = gridDim.x * (unsigned int)nwaves;
         // chosen here: two grabs per wave at least, of at most 64 vertices; but
@@ -1164,15 +1165,15 @@ tc_count_kernel(TcArgs<OffT>)
         // vertices: 450 us, 1040).  A batch's list comes graph by graph.
         unsigned int chunk = a->chunk_wave, fchunk = 1, fronts = 0;
         if (a->chunk_wave <= 0) {
-            chunk = kMode == kModeBatch ? whole : whole - whole / 4;
+            const bool even = kBatch || a->chunk_wave < 0;
+            chunk = even ? whole : whole - whole / 4;
             chunk = max(1u, min((unsigned int)kWave, chunk / (2u * waves)));
             fchunk = max(1u, min(chunk, whole / (16u * waves)));
-            fronts = kMode == kModeBatch ? 0 : whole / (4u * fchunk);
+            fronts = even ? 0 : whole / (4u * fchunk);
         }
         const unsigned int front = extra + fronts * fchunk;  // where the others begin
         const unsigned int n = rank_chunks(
             extra + fronts + ((unsigned int)items - front + chunk - 1u) / chunk, 1, a->rank, a->nranks);
-        constexpr bool kBatch = kMode == kModeBatch;
         constexpr int kShards = kBatch ? kXcds : kWaveShards;
         const bool fixed = !kBatch && n <= gridDim.x * (unsigned int)nwaves;
         unsigned int shard = kBatch ? (unsigned int)xcc_id() : blockIdx.x % kShards;
@@ -1185,7 +1186,7 @@ tc_count_kernel(TcArgs<OffT>)
             const long long lb = a->ctl->list_begin[kTierWave], le = a->ctl->list_begin[kTierWave + 1];
             const unsigned int c = j * (unsigned int)a->nranks + (unsigned int)a->rank;
             unsigned int at = c, step = 1;
-            if (c >= extra + fronts) {
+            if (kBatch || c >= extra + fronts) {
                 at = front + (c - extra - fronts) * chunk;
                 step = chunk;
             } else if (c >= extra) {

@@ -32,8 +32,11 @@
 //  * Persistent workgroups pull chunks of vertices from per-tier atomic
 //    queues (the reference's G_INDEX counters, TC.cu:405-422,560-577);
 //    logical rank r of P takes chunks c with c % P == r (TC.cu:259,433).
-//  * The count is reduced per wave in registers and added once per wave to
-//    a uint64 in device memory (TC.cu:586-596).
+//  * Short rows of the wave tier are counted up to 64 at a time over one
+//    shared table (packs); vertices of long walks in parts (tc_kernels.h).
+//  * The count is reduced per wave in registers, per workgroup in LDS, and
+//    added once per workgroup to one of 16 lines in device memory
+//    (TC.cu:586-596).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -293,7 +293,7 @@ bool walk_index_binned(const Ctx *ctx);
 // Dense core (core.hip).  core_config: the core a count with p asks for
 // (K = 0: none); core_build: the index for ctx->core.want_K/want_thr
 // (synchronises once); core_enqueue: the counting launch, adding to
-// the first of ctl->sums; core_drop: forget the index.
+// ctl->sums; core_drop: forget the index.
 void core_config(const Ctx *ctx, const trust_params &p, int *K, int *thr, bool *automatic);
 int core_build(Ctx *ctx);
 int core_enqueue(Ctx *ctx, TcCtl *ctl, hipStream_t s);

@@ -52,6 +52,7 @@
 #include <cstring>
 #include <vector>
 
+#include "core_items.h"
 #include "engine.h"
 #include "wave_ops.h"
 
@@ -71,7 +72,6 @@ constexpr int kCoreSteps = 6;        // closure steps
 constexpr int kCoreMinDegreeLow = 64, kCoreMinDegreeHigh = 384, kCorePerDegree = 48;
 constexpr int kCoreSample = 128;     // in-degree sampled every 128th entry
 constexpr int kCoreBins = 2048;      // histogram: est < 64 exact, then 64 bins per octave
-constexpr int kCorePart = 2048;      // dense targets per work item (longer lists are cut)
 constexpr int kCoreThreads = 256;
 constexpr int kCoreQueueStride = 32; // one 128-byte line per slice queue
 // misc words: the slice queues follow at 64
@@ -760,8 +760,8 @@ static int core_build_t(Ctx *ctx)
     }
     const int thr = (int)h[kCmDegree];
     c.thr = thr;
-    c.cap = E / std::max(thr, 1) + E / kCorePart + 2;
     c.nsrc_cap = std::max<long long>(h[kCmOver], 1);
+    c.cap = core_item_slots(c.nsrc_cap, E);
     const unsigned members = h[kCmMembers];
     // bit rows: S slices of wd words, wd a power of two in [4, 32]: a slice
     // row is at most one 128-byte line (a lane reads 16 bytes of it)

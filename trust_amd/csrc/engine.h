@@ -62,6 +62,9 @@ struct CsrViews {
     // ids of the hash and probe rows are below this
     int64_t ids = int64_t(1) << 31;
     int64_t entries = 0;  // of the walk rows (0: not known; an upper bound will do)
+    // the walk rows are a built index, whose rows keep no order of entries
+    // from one build to the next
+    bool built = false;
 };
 
 // Shape of one counting launch.

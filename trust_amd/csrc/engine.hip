@@ -283,8 +283,11 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
                         (rc = ctx->block_counts.ensure(kPlanScratch))))
         return rc;
     // a list made elsewhere, and the instrumented mode's per-vertex outputs,
-    // know whole vertices only
-    const bool whole = preplanned || seg || (mode & ~kProbeDeep) == kModeInstr;
+    // know whole vertices only; and ranks that share a count may each have
+    // built a walk index, whose rows hold their entries in another order with
+    // each build: a vertex's parts would then not be the same on all of them
+    const bool whole = preplanned || seg || (mode & ~kProbeDeep) == kModeInstr ||
+                       (views.built && p.total_process > 1);
     const int part_entries = whole ? 0 : walk_part_entries(views.entries);
     const int wave_part = whole ? 0 : walk_wave_part(views.entries, V);
     if (L.spill_groups > 0) {
@@ -791,6 +794,7 @@ int enqueue_resident(Ctx *ctx, const trust_params &p, int mode, const ResidentRu
         v.begW = ctx->side_beg.p;
         v.adjW = nullptr;
         v.entW = ctx->side_ent.p;
+        v.built = true;
         if (ctx->side_entries >= 0)
             v.entries = ctx->side_entries;
     } else if (R.starts) {  // walk rows = N+, each entry's list read from the start index

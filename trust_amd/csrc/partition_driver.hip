@@ -586,12 +586,14 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
                         (const int32_t *)w.out_ids.p, tp.beg.p, (const int32_t *)tp.adj.p};
             vo.entries = w.x_out;
             vo.ids = ids;
+            vo.built = true;
             if ((rc = count_view(vo, rows_of[ji], (TcCtl *)ctls.p + 2 * job)))
                 return rc;
             CsrViews vi{tp.beg.p, (const int32_t *)tp.adj.p, w.in_beg.p,
                         (const int32_t *)w.in_ids.p, th.beg.p, (const int32_t *)th.adj.p};
             vi.entries = w.x_in;
             vi.ids = ids;
+            vi.built = true;
             if ((rc = count_view(vi, rows_of[jk], (TcCtl *)ctls.p + 2 * job + 1)))
                 return rc;
         } else {

@@ -244,6 +244,8 @@ constexpr double kShortWalkShare = 0.45;
 // part_entries is 1/16384 of the walk, so that no part outlasts the count's
 // average workgroup and the list holds at most kGroupExtra more positions; at
 // least 128, below which building the table costs more than the part's walk.
+// Parts cut a row by position, so a rank's share of a count has none where its
+// walk is a built index (each build leaves a row's entries in another order).
 constexpr int kBigPartLg = 2;
 constexpr long long kGroupExtra = 16384;
 inline int walk_part_entries(long long walk_entries)

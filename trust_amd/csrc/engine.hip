@@ -21,8 +21,12 @@
 
 namespace trust {
 
+// Reported here, so not again: the runtime keeps the last error until it is
+// asked for it, and the next launch's check would take it for its own (a count
+// after a failed allocation, or the smaller allocation tried instead).
 int hip_fail(hipError_t e, const char *what)
 {
+    (void)hipGetLastError();
     if (e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation)
         return fail(TRUST_ERR_OOM, "%s: %s", what, hipGetErrorString(e));
     return fail(TRUST_ERR_HIP, "%s: %s", what, hipGetErrorString(e));

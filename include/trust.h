@@ -110,7 +110,7 @@ typedef struct trust_params {
      * core_min_degree: 0 automatic (a 48th of the core's vertices, 64 to 384),
      * else >= 2. */
     int32_t reserved[3];   /* reserved[0]: a tile stream's device tile-cache slots (0: every tile
-                              when they take at most 32 GB, else 2n+2) */
+                              when they take at most 32 GB and fit, else 2n+2) */
     int32_t core_vertices;
     int32_t core_min_degree;
 } trust_params;

@@ -240,16 +240,17 @@ static int journal_add(Journal &jr, long long id, int n, unsigned long long c, u
 }
 
 // Streams all jobs of an n x n partition; tiles[i*n+j] is tile (i,j).
-// cache_slots: tiles held on the device (0: all of them when they are small,
-// else 2n + 2, enough to prefetch).
+// cache_slots: tiles held on the device (0: 2n + 2, enough to prefetch);
+// keep_all: all of them, with the walks' buffers sized for the largest tile.
 // job_counts (nullable, n^3 entries) receives each job's count.  With a
 // journal path, jobs already in the journal are skipped and each new job is
 // appended as its count lands; max_new_jobs > 0 stops after that many new
-// jobs, and *remaining (nullable) receives the jobs still missing.
+// jobs, and *remaining (nullable) receives the jobs still missing.  *added
+// receives the jobs appended, also when the stream fails.
 static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_params &p,
-                        int cache_slots, uint64_t *job_counts, trust_result *r,
-                        const char *journal = nullptr, long long max_new_jobs = 0,
-                        long long *remaining = nullptr)
+                        int cache_slots, bool keep_all, uint64_t *job_counts, trust_result *r,
+                        const char *journal, long long max_new_jobs, long long *remaining,
+                        long long *added)
 {
     const long long njobs = (long long)n * n * n;
     bool off64 = (p.flags & TRUST_FLAG_OFFSETS64) != 0;
@@ -307,18 +308,11 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
     // are parts of one allocation.
     const size_t beg_bytes = ((off64 ? 8 : 4) * (size_t)(maxV + 1) + 255) & ~(size_t)255;
     const size_t adj_bytes = (sizeof(int32_t) * (size_t)std::max<int64_t>(maxE, 1) + 255) & ~(size_t)255;
-    // Unless the caller chose, all tiles stay when they take at most 32 GB
-    // of the 288: each is then copied once, not once for every row of jobs.
     const size_t slot_bytes = beg_bytes + adj_bytes;
-    const bool keep_all = cache_slots <= 0 && slot_bytes * (size_t)n * (size_t)n <= (32ull << 30);
-    const int few = std::max(3, std::min(cache_slots > 0 ? cache_slots : 2 * n + 2, n * n));
-    cache_slots = keep_all ? std::max(3, n * n) : few;
+    cache_slots = std::max(3, keep_all ? n * n
+                                       : std::min(cache_slots > 0 ? cache_slots : 2 * n + 2, n * n));
     DevBuf slab;
     rc = slab.ensure(slot_bytes * (size_t)cache_slots);
-    if (rc == TRUST_ERR_OOM && cache_slots > few) {
-        cache_slots = few;
-        rc = slab.ensure(slot_bytes * (size_t)cache_slots);
-    }
     if (rc)
         return rc;
     std::vector<TileSlot> slots((size_t)cache_slots);
@@ -374,14 +368,16 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
     std::vector<int> walk_row(walks.size(), -1);  // the tile row i each walk was built for
     if (short_walk && keep_all) {
         // the walks' buffers for the largest tile at once: growing one frees
-        // it, which waits for the device (without room they are sized as
-        // they are needed)
+        // it, which waits for the device
         const size_t ob = off64 ? 8 : 4, most = sizeof(int32_t) * (size_t)std::max<int64_t>(maxE, 1);
-        bool room = !ctx->wi.recs.ensure(2 * most) && !ctx->wi.rel.ensure(most) &&
-                    !ctx->side_cnt.ensure(2 * sizeof(int) * (size_t)std::max<int64_t>(maxV, 1));
+        if ((rc = ctx->wi.recs.ensure(2 * most)) || (rc = ctx->wi.rel.ensure(most)) ||
+            (rc = ctx->side_cnt.ensure(2 * sizeof(int) * (size_t)std::max<int64_t>(maxV, 1))))
+            return rc;
         for (TileWalk &w : walks)
-            room = room && !w.out_ids.ensure(most) && !w.in_ids.ensure(most) &&
-                   !w.out_beg.ensure(ob * (size_t)(maxV + 1)) && !w.in_beg.ensure(ob * (size_t)(maxV + 1));
+            if ((rc = w.out_ids.ensure(most)) || (rc = w.in_ids.ensure(most)) ||
+                (rc = w.out_beg.ensure(ob * (size_t)(maxV + 1))) ||
+                (rc = w.in_beg.ensure(ob * (size_t)(maxV + 1))))
+                return rc;
     }
     if (short_walk) {
         // global out-degree of every vertex, class by class (sum over its tile row)
@@ -449,6 +445,7 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
             if (int rc2 = journal_add(jr, job, n, c, w))
                 return rc2;
             journaled++;
+            ++*added;
         }
         return TRUST_OK;
     };
@@ -710,6 +707,42 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
     return TRUST_OK;
 }
 
+// Unless the caller chose the slots, all tiles stay on the device when they
+// take at most 32 GB of the 288: each is then copied once, not once for every
+// row of jobs.  Where the device has no room for that, at any point of the
+// stream, everything is given back and the stream starts again with 2n + 2
+// slots and walk buffers of the sizes needed (a journal keeps what it has).
+static int count_tiles(const trust_csr *tiles, int n, const trust_params &p, uint64_t *job_counts,
+                       trust_result *r, const char *journal, long long max_new_jobs,
+                       long long *remaining)
+{
+    const int slots = p.reserved[0];
+    uint64_t maxV = 0, maxE = 0;
+    bool off64 = (p.flags & TRUST_FLAG_OFFSETS64) != 0;
+    for (int t = 0; t < n * n; t++) {
+        maxV = std::max(maxV, (uint64_t)std::max<int64_t>(tiles[t].vertices, 0));
+        maxE = std::max(maxE, (uint64_t)std::max<int64_t>(tiles[t].edges, 0));
+        off64 = off64 || tiles[t].edges >= kMaxEdges32;
+    }
+    const double all = ((off64 ? 8.0 : 4.0) * ((double)maxV + 1) + 4.0 * (double)maxE) * n * n;
+    bool keep_all = slots <= 0 && all <= (double)(32ull << 30);
+    for (;;) {
+        long long added = 0;
+        Ctx ctx;
+        int rc = ctx_init(&ctx, p.device);
+        if (rc)
+            return rc;
+        rc = stream_tiles(&ctx, tiles, n, p, slots, keep_all, job_counts, r, journal, max_new_jobs,
+                          remaining, &added);
+        if (rc != TRUST_ERR_OOM || !keep_all)
+            return rc;
+        keep_all = false;
+        clear_error();
+        if (max_new_jobs > 0)  // more of them were to come: the last is added after its count
+            max_new_jobs = std::max<long long>(max_new_jobs - added, 1);
+    }
+}
+
 }  // namespace trust
 
 using namespace trust;
@@ -722,11 +755,7 @@ extern "C" int trust_count_tiles(const trust_csr *tiles, int n, const trust_para
     int rc = check_params(*p);
     if (rc)
         return rc;
-    Ctx ctx;
-    rc = ctx_init(&ctx, p->device);
-    if (rc)
-        return rc;
-    return stream_tiles(&ctx, tiles, n, *p, p->reserved[0], nullptr, r);
+    return count_tiles(tiles, n, *p, nullptr, r, nullptr, 0, nullptr);
 }
 
 extern "C" int trust_count_tiles_journal(const trust_csr *tiles, int n, const trust_params *p,
@@ -738,13 +767,8 @@ extern "C" int trust_count_tiles_journal(const trust_csr *tiles, int n, const tr
     int rc = check_params(*p);
     if (rc)
         return rc;
-    Ctx ctx;
-    rc = ctx_init(&ctx, p->device);
-    if (rc)
-        return rc;
     long long remaining = 0;
-    rc = stream_tiles(&ctx, tiles, n, *p, p->reserved[0], job_counts, r, journal, (long long)max_new_jobs,
-                      &remaining);
+    rc = count_tiles(tiles, n, *p, job_counts, r, journal, (long long)max_new_jobs, &remaining);
     if (rc)
         return rc;
     return (int)std::min<long long>(remaining, INT32_MAX);

@@ -446,7 +446,8 @@ static int index_begin(Ctx *ctx, ResidentRun &R)
 // it makes at most kShortWalkShare of the reference walk's probes.  The
 // probe totals and the in-walk rows depend on the graph alone, so a context
 // makes them once per loaded graph (or again under TRUST_FLAG_FRESH_INDEX);
-// the count that makes them includes their device time in its seconds.
+// the count that makes them includes their device time in its seconds.  The
+// choice depends on the graph and the core asked for, not on earlier counts.
 static int prepare_side(Ctx *ctx, bool force, bool starts, ResidentRun &R)
 {
     DevCsr &g = ctx->g;
@@ -520,8 +521,10 @@ static int prepare_side(Ctx *ctx, bool force, bool starts, ResidentRun &R)
         }
     }
     // (of the short walk's probes those that the dense core takes over do not
-    // count)
-    const uint64_t core_probes = ctx->core.active ? ctx->core.dense_probes : 0;
+    // count; where the reference pass goes first the choice is made without a
+    // core, and stays so when a forced short-side walk has built one since)
+    const uint64_t core_probes =
+        ctx->core.active && !walk_probably_reference(ctx) ? ctx->core.dense_probes : 0;
     R.side = force ||
              (double)(ctx->side_w_short - core_probes) <= kShortWalkShare * (double)ctx->side_w_ref;
     if (R.side && !ctx->side_built) {

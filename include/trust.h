@@ -102,10 +102,10 @@ typedef struct trust_params {
      * highest estimated degrees, closed under out-neighbours while it stays
      * within 32768 vertices.  A per-graph index like the walk rows, made by
      * the first count that uses it.  core_vertices: 0 automatic (for single
-     * graphs of at least 9 * 2^20 edges and 14 edges per vertex (11 from 2^25
-     * edges on; 24 * 2^20 and 16 when the call makes and drops its own
-     * context) counted by one logical rank a power of two near twice the
-     * square root of the vertices, at most 16384; else none),
+     * graphs of at least 9 * 2^20 edges and 14 edges per non-empty row (11
+     * from 2^25 edges on; 24 * 2^20 and 16 when the call makes and drops its
+     * own context) counted by one logical rank a power of two near twice the
+     * square root of those rows, at most 16384; else none),
      * -1 none, else a power of two in [256, 16384].
      * core_min_degree: 0 automatic (a 48th of the core's vertices, 64 to 384),
      * else >= 2. */

@@ -46,6 +46,7 @@ struct DevCsr {
     DevBuf beg, adj;
     int64_t V = 0, E = 0;
     int64_t max_deg = 0;
+    int64_t rows = 0;  // that are not empty: what empty rows for unused ids leave alone
     bool off64 = false;
 };
 
@@ -303,8 +304,8 @@ int core_enqueue(Ctx *ctx, TcCtl *ctl, hipStream_t s);
 void core_drop(Ctx *ctx);
 // core_drop and free the core's device memory (a synchronised stream)
 void core_release(Ctx *ctx);
-// A graph whose top out-degree is under 24 times the mean takes the
-// reference walk on every family measured (R-MAT 10-18, Chung-Lu, ER, BA:
+// A graph whose top out-degree is under 24 times the mean (of the rows that
+// are not empty) takes the reference walk on every family measured (R-MAT 10-18, Chung-Lu, ER, BA:
 // 1.8 to 19 times; R-MAT 20 and up, which take the short side: 27 and up);
 // where the dense core is wanted the line is 12 times, since with it dense
 // R-MAT graphs (12 to 23 times) take the short side.

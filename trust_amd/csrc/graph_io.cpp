@@ -95,12 +95,16 @@ int load_folder(const std::string &folder, HostCsr &out)
     return trust_csr_validate(out.beg.data(), out.adj.data(), out.V, out.E);
 }
 
-int64_t host_max_degree(const int64_t *beg, int64_t V)
+int64_t host_max_degree(const int64_t *beg, int64_t V, int64_t *rows)
 {
-    int64_t maxd = 0;
-#pragma omp parallel for reduction(max : maxd)
-    for (int64_t u = 0; u < V; u++)
+    int64_t maxd = 0, some = 0;
+#pragma omp parallel for reduction(max : maxd) reduction(+ : some)
+    for (int64_t u = 0; u < V; u++) {
         maxd = std::max(maxd, beg[u + 1] - beg[u]);
+        some += beg[u + 1] > beg[u];
+    }
+    if (rows)
+        *rows = some;
     return maxd;
 }
 

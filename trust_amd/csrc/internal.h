@@ -32,8 +32,8 @@ int read_file(const std::string &path, void *dst, size_t bytes);
 int write_file(const std::string &path, const void *src, size_t bytes);
 int load_folder(const std::string &folder, HostCsr &out);
 
-// Largest beg[u+1]-beg[u] (OpenMP, host).
-int64_t host_max_degree(const int64_t *beg, int64_t V);
+// Largest beg[u+1]-beg[u] (OpenMP, host); *rows (nullable): rows that are not empty.
+int64_t host_max_degree(const int64_t *beg, int64_t V, int64_t *rows = nullptr);
 
 // memcpy with all OpenMP threads, in 256 KB pieces.
 void host_parallel_copy(void *dst, const void *src, size_t bytes);

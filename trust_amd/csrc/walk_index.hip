@@ -826,7 +826,7 @@ bool walk_probably_reference(const Ctx *ctx)
 {
     const DevCsr &g = ctx->g;
     const double share = ctx->core.want_K ? 12.0 : 24.0;
-    return (double)g.max_deg * (double)g.V < share * (double)g.E;
+    return (double)g.max_deg * (double)g.rows < share * (double)g.E;
 }
 
 int reference_pass(Ctx *ctx, bool starts)

@@ -61,3 +61,23 @@ def test_default_fits_where_few_slots_do(gpu, shape, tmp_path):
         assert T.device_memory_held() == held
     finally:
         T.set_device_memory_cap(0)
+
+
+def test_many_jobs_need_no_block_each(gpu, tmp_path):
+    # 512 jobs of two counts: with a control block kept for each the stream takes 21 MB
+    n = 8
+    beg, adj = T.rmat_csr(18, 16, seed=1)
+    want = oracle.count_hash(beg, adj)
+    tiles = T.partition_csr(beg, adj, n)
+    print("[gpu] 8 x 8 tiles under 13 MB", flush=True)
+    try:
+        T.set_device_memory_cap(T.device_memory_held() + (13 << 20))
+        assert T.count_tiles(tiles, n).triangles == want
+        for jobs in (1, 15, 16, 17):  # around the control blocks' ring
+            journal = str(tmp_path / f"journal{jobs}")
+            missing, _, _ = T.count_tiles_journal(tiles, n, journal, max_new_jobs=jobs)
+            assert missing == n ** 3 - jobs
+            missing, r, each = T.count_tiles_journal(tiles, n, journal)
+            assert (missing, r.triangles, int(each.sum())) == (0, want, want)
+    finally:
+        T.set_device_memory_cap(0)

@@ -144,7 +144,7 @@ int enqueue_segments(Ctx *ctx, const trust_params &p, int mode, const ResidentRu
 {
     const DevCsr &g = ctx->g;
     const int64_t ng = ctx->batch_ngraphs;
-    int rc = ctx->list.ensure(sizeof(int32_t) * (size_t)(g.V + kMaxExtra));
+    int rc = ctx->list.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(g.V, 1));
     if (rc)
         return rc;
     unsigned long long *out = (unsigned long long *)ctx->batch_out.p;

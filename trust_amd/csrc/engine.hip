@@ -283,7 +283,8 @@ int enqueue_count(Ctx *ctx, const CsrViews &views, int64_t V, bool same_csr,
     // a list made elsewhere is in place already: growing the buffer here would
     // drop it
     int rc = TRUST_OK;
-    if (!preplanned && ((rc = ctx->list.ensure(sizeof(int32_t) * (size_t)(V + kMaxExtra))) ||
+    const long long positions = std::max<long long>(V + list_extra(views.entries), 1);
+    if (!preplanned && ((rc = ctx->list.ensure(sizeof(int32_t) * (size_t)positions)) ||
                         (rc = ctx->block_counts.ensure(kPlanScratch))))
         return rc;
     // a list made elsewhere, and the instrumented mode's per-vertex outputs,

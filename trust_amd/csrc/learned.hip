@@ -594,7 +594,7 @@ static int ensure_plan_buffers(Ctx *ctx)
     if ((rc = ctx->feat.ensure(sizeof(float) * 3 * V)) ||
         (rc = ctx->cost.ensure(sizeof(float) * V)) ||
         (rc = ctx->tiers.ensure(sizeof(unsigned short) * V)) ||
-        (rc = ctx->list.ensure(sizeof(int32_t) * (V + kMaxExtra))))
+        (rc = ctx->list.ensure(sizeof(int32_t) * V)))
         return rc;
     return TRUST_OK;
 }

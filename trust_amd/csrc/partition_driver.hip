@@ -7,7 +7,7 @@
 // tiles synchronously each time (TC.cu:1034-1077).  Here all jobs stream
 // through one device: tiles live in a bounded device cache, missing tiles
 // are copied on a second stream while the previous job counts, and each
-// job's uint64 lands in its own control block, summed once at the end.
+// job's totals are kept on the device and summed once at the end.
 #include <hip/hip_runtime.h>
 
 #include <sys/types.h>
@@ -331,7 +331,7 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
     const size_t stage_bytes = ((sizeof(int32_t) * (size_t)maxE + 255) & ~(size_t)255) +
                                sizeof(int64_t) * (size_t)(maxV + 1);
     const bool pinned_uploads = stage.init(stage_bytes);
-    rc = ctx->list.ensure(sizeof(int32_t) * (size_t)(maxV + kMaxExtra));
+    rc = ctx->list.ensure(sizeof(int32_t) * (size_t)(maxV + list_extra(maxE)));
     if (!rc)
         rc = ctx->block_counts.ensure(kPlanScratch);
     if (rc)
@@ -397,9 +397,12 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
             todo.push_back(job);
     if (max_new_jobs > 0 && (long long)todo.size() > max_new_jobs)
         todo.resize((size_t)max_new_jobs);
-    DevBuf ctls;
-    const long long nctl = short_walk ? 2 * njobs : njobs;
+    // The control blocks of kRing jobs at a time; what is kept of each (the
+    // totals) is taken from them when the last of the jobs has been queued.
+    constexpr size_t kRing = 16;
+    DevBuf ctls, totals;
     const int per_job = short_walk ? 2 : 1;  // control blocks per job
+    const size_t nctl = (size_t)per_job * todo.size();
     // journal: each job's control blocks come back to pinned host memory
     // right after its launches, with an event to poll
     TcCtl *hctl = nullptr;
@@ -420,7 +423,8 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
         }
     } journal_guard{hctl, cev, ctx->stream};
     if (journal) {
-        HIPCHK(hipHostMalloc((void **)&hctl, sizeof(TcCtl) * (size_t)nctl, hipHostMallocDefault));
+        HIPCHK(hipHostMalloc((void **)&hctl, sizeof(TcCtl) * std::max<size_t>(nctl, 1),
+                             hipHostMallocDefault));
         cev.assign((size_t)njobs, nullptr);
         for (long long job : todo)
             HIPCHK(hipEventCreateWithFlags(&cev[(size_t)job], hipEventDisableTiming));
@@ -438,9 +442,10 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
                 return hip_fail(e, "journal event");
             unsigned long long c = 0, w = 0;
             for (int q = 0; q < per_job; q++) {
-                fold_ctl(hctl[(size_t)(per_job * job + q)]);
-                c += hctl[(size_t)(per_job * job + q)].count;
-                w += hctl[(size_t)(per_job * job + q)].probes;
+                TcCtl &x = hctl[per_job * journaled + q];
+                fold_ctl(x);
+                c += x.count;
+                w += x.probes;
             }
             if (int rc2 = journal_add(jr, job, n, c, w))
                 return rc2;
@@ -449,8 +454,8 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
         }
         return TRUST_OK;
     };
-    rc = ctls.ensure(sizeof(TcCtl) * (size_t)nctl);
-    if (rc)
+    if ((rc = ctls.ensure(sizeof(TcCtl) * per_job * std::max<size_t>(std::min(kRing, todo.size()), 1))) ||
+        (rc = totals.ensure(sizeof(TcTotals) * std::max<size_t>(nctl, 1))))
         return rc;
 
     // per job: events around its counting launches (the count's share of the
@@ -576,6 +581,7 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
             HIPCHK(hipStreamWaitEvent(ctx->stream, slots[sl[q]].ready, 0));
         }
         const DevCsr &th = slots[sl[0]].g, &tp = slots[sl[2]].g;
+        TcCtl *ctl = (TcCtl *)ctls.p + per_job * (t % kRing);
         HIPCHK(hipEventRecord(jev[(size_t)(2 * job)], ctx->stream));
         if (short_walk) {
             const TileWalk &w = walks[(size_t)jk];
@@ -584,14 +590,14 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
             vo.entries = w.x_out;
             vo.ids = ids;
             vo.built = true;
-            if ((rc = count_view(vo, rows_of[ji], (TcCtl *)ctls.p + 2 * job)))
+            if ((rc = count_view(vo, rows_of[ji], ctl)))
                 return rc;
             CsrViews vi{tp.beg.p, (const int32_t *)tp.adj.p, w.in_beg.p,
                         (const int32_t *)w.in_ids.p, th.beg.p, (const int32_t *)th.adj.p};
             vi.entries = w.x_in;
             vi.ids = ids;
             vi.built = true;
-            if ((rc = count_view(vi, rows_of[jk], (TcCtl *)ctls.p + 2 * job + 1)))
+            if ((rc = count_view(vi, rows_of[jk], ctl + 1)))
                 return rc;
         } else {
             const DevCsr &tw = slots[sl[1]].g;
@@ -599,19 +605,21 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
                        tp.beg.p, (const int32_t *)tp.adj.p};
             v.entries = tw.E;
             v.ids = ids;
-            if ((rc = count_view(v, tiles[cur[0]].vertices, (TcCtl *)ctls.p + job)))
+            if ((rc = count_view(v, tiles[cur[0]].vertices, ctl)))
                 return rc;
         }
         (void)jj;
         HIPCHK(hipEventRecord(jev[(size_t)(2 * job + 1)], ctx->stream));
         if (journal) {
-            const size_t c0 = (size_t)(per_job * job);
-            HIPCHK(hipMemcpyAsync(hctl + c0, (TcCtl *)ctls.p + c0, sizeof(TcCtl) * per_job,
+            HIPCHK(hipMemcpyAsync(hctl + per_job * t, ctl, sizeof(TcCtl) * per_job,
                                   hipMemcpyDeviceToHost, ctx->stream));
             HIPCHK(hipEventRecord(cev[(size_t)job], ctx->stream));
             if ((rc = journal_ready(false)))
                 return rc;
         }
+        if (t % kRing == kRing - 1 || t + 1 == todo.size())
+            HIPCHK(launch_totals((const TcCtl *)ctls.p, (int)(per_job * (t % kRing + 1)),
+                                 (TcTotals *)totals.p + per_job * (t - t % kRing), ctx->stream));
         for (int q = 0; q < 3; q++)
             if (sl[q] >= 0)
                 HIPCHK(hipEventRecord(slots[sl[q]].released, ctx->stream));
@@ -632,31 +640,23 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
         }
     }
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-    std::vector<TcCtl> h((size_t)nctl);
-    HIPCHK(hipMemcpyAsync(h.data(), ctls.p, sizeof(TcCtl) * (size_t)nctl, hipMemcpyDeviceToHost,
-                          ctx->stream));
+    std::vector<TcTotals> h(nctl);
+    if (nctl > 0)
+        HIPCHK(hipMemcpyAsync(h.data(), totals.p, sizeof(TcTotals) * nctl, hipMemcpyDeviceToHost,
+                              ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    for (TcCtl &x : h)
-        fold_ctl(x);
-    if (short_walk)  // fold each job's in-walk count into its out-walk count
-        for (long long j : todo) {
-            TcCtl &a = h[(size_t)(2 * j)];
-            const TcCtl &b = h[(size_t)(2 * j + 1)];
-            a.count += b.count;
-            a.probes += b.probes;
-            a.rebuilds += b.rebuilds;
-        }
     if (journal && (rc = journal_ready(true)))
         return rc;
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
     double count_s = 0;
-    std::vector<char> counted((size_t)njobs, 0);
-    for (long long j : todo) {
+    std::vector<long long> counted((size_t)njobs, -1);  // a job's place in todo
+    for (size_t t = 0; t < todo.size(); t++) {
+        const long long j = todo[t];
         float jm = 0;
         HIPCHK(hipEventElapsedTime(&jm, jev[(size_t)(2 * j)], jev[(size_t)(2 * j + 1)]));
         count_s += jm * 1e-3;
-        counted[(size_t)j] = 1;
+        counted[(size_t)j] = (long long)t;
     }
     double build_s = 0;
     for (int b = 0; b < nbuilds; b++) {
@@ -668,11 +668,13 @@ static int stream_tiles(Ctx *ctx, const trust_csr *tiles, int n, const trust_par
     long long missing = 0;
     for (long long j = 0; j < njobs; j++) {
         uint64_t c = 0;
-        if (counted[(size_t)j]) {  // this call
-            const TcCtl &x = h[(size_t)(short_walk ? 2 * j : j)];
-            c = x.count;
-            probes += x.probes;
-            rebuilds += x.rebuilds;
+        if (counted[(size_t)j] >= 0) {  // this call
+            for (int q = 0; q < per_job; q++) {
+                const TcTotals &x = h[(size_t)(per_job * counted[(size_t)j] + q)];
+                c += x.count;
+                probes += x.probes;
+                rebuilds += x.rebuilds;
+            }
         } else if (journal && jr.have[(size_t)j]) {  // an earlier call
             c = jr.cnt[(size_t)j];
             probes += jr.prb[(size_t)j];

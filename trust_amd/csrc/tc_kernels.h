@@ -166,7 +166,7 @@ struct PlanArgs {
     int wave_only;
     int part_entries;   // see group_parts (0: vertices stay whole)
     int wave_part;      // see wave_parts
-    int32_t *list;      // V + kMaxExtra positions
+    int32_t *list;      // V + list_extra(walk entries) positions
     int *block_counts;  // kPlanBlocks x 2 kNumTiers
     int per_block;      // set by launch_plan
     TcCtl *ctl;
@@ -174,7 +174,14 @@ struct PlanArgs {
 
 constexpr size_t kPlanScratch = sizeof(int) * 2 * kNumTiers * kPlanBlocks;  // PlanArgs::block_counts
 
+// What a stream of many counts keeps of each control block.
+struct TcTotals {
+    unsigned long long count, probes, rebuilds;
+};
+
 // Launch wrappers (tc_kernels.hip).  All launches go on `stream`.
+// totals[i] = those of ctl[i], i < n
+hipError_t launch_totals(const TcCtl *ctl, int n, TcTotals *totals, hipStream_t stream);
 template <typename OffT>
 hipError_t launch_plan(PlanArgs<OffT> p, hipStream_t stream);
 template <typename OffT>
@@ -292,7 +299,14 @@ __host__ __device__ inline int wave_parts(int dW, int each)
     const int n = (dW + each - 1) / each;
     return n < kMaxWaveParts ? n : kMaxWaveParts;
 }
-constexpr long long kMaxExtra = kGroupExtra + kWaveExtra;  // list positions beyond one per vertex
+// List positions beyond one per vertex, for walks of up to `entries` entries:
+// a vertex fills fewer than one per part's entries.
+constexpr long long kMaxExtra = kGroupExtra + kWaveExtra;
+inline long long list_extra(long long entries)
+{
+    const long long g = entries >> 7, w = entries >> 4;
+    return (g < kGroupExtra ? g : kGroupExtra) + (w < kWaveExtra ? w : kWaveExtra);
+}
 
 // Packs of the wave tier (tc_kernels.hip): ids below `ids` leave the upper
 // bits of a 32-bit key for the row's number; the largest number is left out,

@@ -1727,7 +1727,29 @@ __global__ void fill_u32_kernel(uint32_t *dst, uint32_t value, long long n)
         dst[i] = value;
 }
 
+__global__ void totals_kernel(const TcCtl *__restrict__ ctl, int n, TcTotals *__restrict__ totals)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n)
+        return;
+    TcTotals t = {ctl[i].count, ctl[i].probes, ctl[i].rebuilds};
+    for (int k = 0; k < kSumLines; k++) {
+        t.count += ctl[i].sums[k].count;
+        t.probes += ctl[i].sums[k].probes;
+    }
+    totals[i] = t;
+}
+
 // ------------------------------------------------------------- wrappers
+hipError_t launch_totals(const TcCtl *ctl, int n, TcTotals *totals, hipStream_t stream)
+{
+    if (n <= 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(totals_kernel, dim3((unsigned)(n + 63) / 64), dim3(64), 0, stream, ctl, n,
+                       totals);
+    return hipGetLastError();
+}
+
 template <typename OffT>
 hipError_t launch_plan(PlanArgs<OffT> p, hipStream_t stream)
 {

@@ -1144,7 +1144,8 @@ tc_count_kernel(TcArgs<OffT>)
         // reference's interleave.  A single large graph interleaves the
         // shards, which spreads each vertex range over all eight L2s (R-MAT
         // 26: contiguous shards measured up to 3% slower).  A batch's list
-        // is in graph order: its shards are contiguous eighths, one for the
+        // is in graph order (the further parts of all graphs, if any, then
+        // the vertices of all): its shards are contiguous eighths, one for the
         // workgroups of each XCD (dealt round-robin), so the graphs that an
         // XCD counts at a time stay in its L2 (10k-graph ER/BA batch: 4.8%
         // faster; four parts per XCD measured 17% slower than one).
@@ -1155,7 +1156,8 @@ tc_count_kernel(TcArgs<OffT>)
         // The tier's list holds the parts beyond a vertex's first (wave_parts),
         // each a chunk of its own, then every vertex (its first part).
         const long long items = a->ctl->list_begin[kTierWave + 1] - a->ctl->list_begin[kTierWave];
-        constexpr bool kBatch = kMode == kModeBatch;  // whole vertices, chunks alike
+        // (a batch's further parts are positions like the others)
+        constexpr bool kBatch = kMode == kModeBatch;
         const unsigned int extra = kBatch ? 0u : (unsigned int)a->ctl->extra[kTierWave];
         const unsigned int whole = (unsigned int)items - extra;
         const unsigned int waves = gridDim.x * (unsigned int)nwaves;
@@ -1165,7 +1167,7 @@ tc_count_kernel(TcArgs<OffT>)
         // that took 10 to 64 of the longest at once ended last: R-MAT 18
         // 775 us, now 570; R-MAT 22 with int64 offsets 2.65 ms, now 2.22.
         // Single vertices all along cost what packs give (Chung-Lu, 3.8 M
-        // vertices: 450 us, 1040).  A batch's list comes graph by graph.
+        // vertices: 450 us, 1040).  A batch's vertices come graph by graph.
         unsigned int chunk = a->chunk_wave, fchunk = 1, fronts = 0;
         if (a->chunk_wave <= 0) {
             const bool even = kBatch || a->chunk_wave < 0;
